@@ -20,18 +20,28 @@
 #pragma once
 #include "minp_bound.h"
 #include "sampler_kernels.h"
+#include "select_bins.h"
 
 namespace rl {
 
 struct FullRow {
     float M;           // the f32::max fold of the penalised row
-    uint32_t done;     // the row is finished (no finite maximum, or the min-p path)
+    uint32_t done;     // the row is finished (no finite maximum, the min-p path, or the selection path)
+    uint32_t thr;      // the last bin k_full_gather collects, or SEL_NONE
+    float R;           // the bins' reference value
+    uint32_t count;    // elements in bins 0..thr
+    uint32_t groups;   // groups they are sorted in
+    uint32_t binned;   // the row was counted into bins (they are cleared by k_full_head)
 };
 
+// Most chunks of a row on the full path: one lane of a wave each. A launch with
+// selection rows uses them all while rows are few; the min-p path's rows, whose
+// last chunk goes through every chunk's candidates, are read in MAX_CHUNKS.
+constexpr uint32_t FULL_CHUNKS = 64;
 // Candidates the min-p path collects per row (a superset of the survivors).
 constexpr uint32_t SURV_CAP = 4096;
 // A row's per-chunk results are read one chunk per lane.
-static_assert(MAX_CHUNKS <= WAVE, "a wave holds one lane per chunk");
+static_assert(FULL_CHUNKS <= WAVE && MAX_CHUNKS <= FULL_CHUNKS, "a wave holds one lane per chunk");
 
 struct FullScratch {
     uint32_t *keyA, *idA, *keyB, *idB;  // [slot][vocab] k_full_rest: the sort's passes
@@ -41,7 +51,16 @@ struct FullScratch {
     double *psum;                       // [slot][chunk] k_full_pass: its mass
     uint64_t *surv;                     // [slot][SURV_CAP] min-p candidates (composites), a region per chunk
     FullRow *row;                       // [slot]
-    uint32_t *arrive;                   // [slot] k_full_pass: chunks done; zero between calls
+    uint32_t *arrive;                   // [slot] workgroups done; zero between kernels
+    // The selection path (full_select.h).
+    uint32_t pass_chunks, gather_chunks;  // the grids of k_full_pass and k_full_gather
+    uint32_t *sel_cnt;                  // [slot][SEL_BINS] elements per bin; zero between calls
+    uint32_t *sel_mass;                 // [slot][SEL_BINS] their mass (SEL_MASS_ONE); zero between calls
+    uint32_t *sel_off;                  // [slot][SEL_GROUPS + 1] where each group starts
+    uint32_t *sel_fill;                 // [slot][SEL_GROUPS] elements a group has been given; zero between calls
+    uint32_t *sel_n;                    // [slot][FULL_CHUNKS] k_full_gather: a short head's elements per chunk
+    double *sel_tail;                   // [slot][FULL_CHUNKS] the chunk's p outside the head
+    uint64_t *sel_rec;                  // [slot][SEL_GROUPS][4] the sorted groups' statistics
 };
 
 constexpr uint32_t SEQ_ITEMS = 8;          // terms per thread per tile of the sum replay
@@ -60,8 +79,8 @@ __device__ __forceinline__ bool identity_order(const rl_sampling &s, uint32_t V)
 
 // Chunk c of n items split into `chunks`: [chunk_lo(c), chunk_lo(c + 1)).
 // Callers split a row's float4 (n <= 2^19, the vocabulary being at most 2^21)
-// into at most MAX_CHUNKS, so n * c fits 32 bits.
-static_assert((uint64_t)MAX_CHUNKS * (1u << 19) < (1ull << 32), "chunk bounds in 32 bits");
+// into at most FULL_CHUNKS, so n * c fits 32 bits.
+static_assert((uint64_t)FULL_CHUNKS * (1u << 19) < (1ull << 32), "chunk bounds in 32 bits");
 __device__ __forceinline__ uint32_t chunk_lo(uint32_t n, uint32_t c, uint32_t chunks) {
     return n * c / chunks;
 }
@@ -87,6 +106,13 @@ struct TempScale {
 // candidates (top_k 0 or >= vocab), sampling (not greedy).
 __device__ __forceinline__ bool small_eligible(const rl_sampling &s, uint32_t V) {
     return s.min_p > 0.0f && full_k(s, V) == V && s.temperature > 0.0f;
+}
+
+// Whether a row takes the selection path (full_select.h): it keeps the head of
+// the descending order, by top-k (top_k < vocab), or by top-p alone over the
+// whole vocabulary (with min-p on it tries the min-p path).
+__device__ __forceinline__ bool select_eligible(const rl_sampling &s, uint32_t V) {
+    return s.temperature > 0.0f && (full_k(s, V) < V || (s.top_p < 1.0f && !(s.min_p > 0.0f)));
 }
 
 // LDS bytes of a chunk's window bitmap: one bit per element of the largest
@@ -398,7 +424,10 @@ __host__ __device__ inline size_t k_full_pass_lds_bytes(uint32_t vocab, uint32_t
 // min-p path also get, per chunk, the mass relative to the chunk's maximum
 // and the candidates that could survive min-p (appended to the row's list),
 // and the last chunk finishes them when it can (done = 1).
-template <bool VEC>
+// With SEL (some row of the launch takes the selection path), such rows'
+// elements are also counted into the row's bins, with their mass, for
+// k_full_gather, which takes such rows from there.
+template <bool VEC, bool SEL>
 __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScratch f) {
     extern __shared__ __align__(16) uint8_t smem[];
     RL_LDS uint32_t *bm = (RL_LDS uint32_t *)smem;  // window ids in this chunk, one bit per element
@@ -411,7 +440,9 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
     __shared__ uint64_t exp_tab[32];
     __shared__ uint64_t cbuf[PASS_CAND];  // this chunk's candidates, filtered by its maximum at the end
     __shared__ uint32_t sh_cn, sh_cover;
-    __shared__ uint32_t red_cnt[MAX_CHUNKS];   // the finisher: each chunk's listed candidates
+    __shared__ uint32_t red_cnt[FULL_CHUNKS];   // the finisher: each chunk's listed candidates
+    __shared__ uint32_t bin_cnt[SEL ? SEL_BINS : 1];  // the chunk's bins
+    __shared__ uint32_t bin_mass[SEL ? SEL_BINS : 1];
     const uint32_t slot = blockIdx.y, chunk = blockIdx.x;
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / WAVE;
     const uint32_t row = a.rows ? a.rows[slot] : a.row0 + slot;
@@ -449,6 +480,15 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
         }
     }
     const uint64_t tab = EXP2_32_TAB[tid & 31u];
+    float ref = -__builtin_inff();  // the sample's maximum (SEL)
+    if constexpr (SEL) {
+        static_assert(SEL_SAMPLE == 4 * FULL_THREADS, "four samples a thread");
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint32_t e = k * FULL_THREADS + tid;
+            ref = fmaxf(ref, ((const RL_GLB float *)rowp)[e < V ? e : V - 1]);
+        }
+    }
     f32x4 A[PASS_U];
     // Buffer loads need no guard (past the row they return zeros); a uniform
     // branch here would also make the compiler wait for all loads at its end.
@@ -484,7 +524,23 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
         sh_cover = 0;
     }
     if (tid < 32) exp_tab[tid] = tab;  // for the finisher
+    const bool select = SEL && select_eligible(s, V);
+    if constexpr (SEL) {
+        ref = wave_maxnum_f32(ref);
+        if (lane == 0) red_m[wave] = ref;
+        if (select)
+            for (uint32_t i = tid; i < SEL_BINS; i += FULL_THREADS) {
+                bin_cnt[i] = 0;
+                bin_mass[i] = 0;
+            }
+    }
     __syncthreads();
+    if constexpr (SEL) {
+        for (uint32_t w = 0; w < FULL_WAVES; ++w) ref = fmaxf(ref, red_m[w]);
+        // + 0: a reference of -0 would part the two zeros' bins from the rest of the order.
+        ref = uniform_f32((ref > -__builtin_inff() && ref < __builtin_inff() ? ref : 0.0f) + 0.0f);
+        __syncthreads();  // red_m is written again at the chunk's end
+    }
     const bool eligible = small_eligible(s, V);
     // Workgroup constants, kept in scalar registers.
     const double invT_d = uniform_f64(1.0 / (double)s.temperature);
@@ -535,6 +591,15 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
             cbuf[at++] = composite(total_key(value_at(e)), e);
         }
     };
+    // Counts element x into its bin (select rows).
+    auto count = [&](float x) {
+        float edge;
+        const uint32_t b = sel_bin(x, ref, &edge);
+        __hip_atomic_fetch_add((RL_LDS uint32_t *)&bin_cnt[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_add((RL_LDS uint32_t *)&bin_mass[b],
+                               (uint32_t)(SEL_MASS_ONE * __builtin_amdgcn_exp2f(-edge * c2)), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
     // A step's PASS_U float4 per thread are all in flight at once (a chunk
     // of the 64-row workload is one step); the penalty is applied in place.
     for (uint32_t b = q0; b < q1; b += PASS_STEP) {
@@ -557,6 +622,15 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
                 }
             }
             if (qq < q1) tmax = fmaxf(tmax, fmaxf(fmaxf(A[u].x, A[u].y), fmaxf(A[u].z, A[u].w)));
+        }
+        if constexpr (SEL) {
+            if (select) {
+#pragma unroll
+                for (uint32_t u = 0; u < PASS_U; ++u)
+                    if (b + u * FULL_THREADS + tid < q1)
+#pragma unroll
+                        for (uint32_t c = 0; c < 4; ++c) count(A[u][c]);
+            }
         }
         tmax = uniform_f32(wave_maxnum_f32(tmax));
         if (tmax > m_run) {
@@ -633,6 +707,7 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
         if (ok) {
             xe = ((const RL_GLB float *)rowp)[e];
             if (pen && ((bm[(e - e0) >> 5] >> ((e - e0) & 31)) & 1u)) xe = penalize(xe, s.repeat_penalty);
+            if (select) count(xe);
         }
         const float tmax = uniform_f32(wave_maxnum_f32(xe));
         if (tmax > m_run) {
@@ -731,6 +806,22 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
                                __HIP_MEMORY_SCOPE_AGENT);
         }
     }
+    if constexpr (SEL) {
+        // A selection row: the chunk's bins into the row's (the barrier after
+        // the waves' records stands between the counting and this).
+        // k_full_gather goes on from there.
+        if (select) {
+            for (uint32_t i = tid; i < SEL_BINS; i += FULL_THREADS)
+                if (bin_cnt[i] != 0) {
+                    __hip_atomic_fetch_add(f.sel_cnt + (uint64_t)slot * SEL_BINS + i, bin_cnt[i], __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_fetch_add(f.sel_mass + (uint64_t)slot * SEL_BINS + i, bin_mass[i], __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+                }
+            if (chunk == 0 && tid == 0) f.row[slot].R = ref;
+            return;
+        }
+    }
     __builtin_amdgcn_s_waitcnt(WAITCNT_VM0);  // this wave's stores have completed
     __syncthreads();                          // and every other wave's
     if (tid == 0) sh_last = atomicAdd(&f.arrive[slot], 1u) == C - 1 ? 1u : 0u;
@@ -773,10 +864,11 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
     if (tid == 0) f.arrive[slot] = 0;  // ready for the next call
     const bool finite = M > -__builtin_inff() && M < __builtin_inff();
     if (!finite || !eligible) {
+        FullRow st{};
+        st.M = M;
+        st.done = finite ? 0u : 1u;
+        st.thr = SEL_NONE;
         if (tid == 0) {
-            FullRow st{};
-            st.M = M;
-            st.done = finite ? 0u : 1u;
             f.row[slot] = st;
             // sample.rs:270-277: argmax, no draw; the first +inf, or 0 when
             // nothing is above -inf.
@@ -858,6 +950,7 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
         FullRow st{};
         st.M = M;
         st.done = fin ? 1u : 0u;
+        st.thr = SEL_NONE;
         f.row[slot] = st;
     }
 }

@@ -1,5 +1,5 @@
-// The FULL path's second launch, k_full_rest: one workgroup per row that
-// k_full_pass left unfinished. It puts the row's candidates in the reference's
+// The FULL path's last launch, k_full_rest: one workgroup per row that the
+// kernels before it (k_full_pass, k_full_head) left unfinished. It puts the row's candidates in the reference's
 // order (descending penalised logit, ascending id; sample.rs:279-305) with a
 // stable LSD radix sort whose passes are chosen by one histogram read, computes
 // p = exp((l - max) / T) as the last pass writes each candidate in place
@@ -15,7 +15,7 @@
 // pick). A row the pass finished exits at once, so a call whose rows all
 // finished in the pass costs one empty launch here.
 #pragma once
-#include "full_kernels.h"
+#include "full_head.h"
 
 namespace rl {
 
@@ -91,53 +91,6 @@ __device__ __forceinline__ void bstore(__amdgpu_buffer_rsrc_t r, uint32_t byte_o
     __builtin_amdgcn_raw_buffer_store_b32(v, r, byte_off, 0, 0);
 }
 
-// ------------------------------------------------------ block helpers ---
-template <uint32_t NT>
-__device__ __forceinline__ uint32_t block_sum_u32(uint32_t v, RL_LDS uint32_t *red) {
-    v = wave_sum_u32(v);
-    __syncthreads();
-    if (lane_id() == 0) red[threadIdx.x / WAVE] = v;
-    __syncthreads();
-    uint32_t t = 0;
-    for (uint32_t w = 0; w < NT / WAVE; ++w) t += red[w];
-    return t;
-}
-
-template <uint32_t NT>
-__device__ __forceinline__ int64_t block_max_i64(int64_t v, RL_LDS int64_t *red) {
-    v = (int64_t)wave_fold_u64((uint64_t)v, [](uint64_t a, uint64_t b) { return (int64_t)a > (int64_t)b ? a : b; });
-    __syncthreads();
-    if (lane_id() == 0) red[threadIdx.x / WAVE] = v;
-    __syncthreads();
-    int64_t t = red[0];
-    for (uint32_t w = 1; w < NT / WAVE; ++w) t = red[w] > t ? red[w] : t;
-    return t;
-}
-
-// Exclusive prefix of v over the workgroup's threads in thread order; *total
-// gets the sum. For doubles it is only used where every partial sum is exact.
-template <uint32_t NT, class T>
-__device__ __forceinline__ T block_exclusive(T v, RL_LDS T *red, T *total) {
-    const uint32_t lane = lane_id(), wave = threadIdx.x / WAVE;
-    T incl;
-    if constexpr (std::is_same<T, double>::value) {
-        incl = wave_incl_f64(v);
-    } else {
-        static_assert(std::is_same<T, uint32_t>::value, "u32 or f64");
-        incl = wave_incl_u32(v);
-    }
-    __syncthreads();
-    if (lane == WAVE - 1) red[wave] = incl;
-    __syncthreads();
-    T before = 0, all = 0;
-    for (uint32_t w = 0; w < NT / WAVE; ++w) {
-        if (w < wave) before += red[w];
-        all += red[w];
-    }
-    *total = all;
-    return before + incl - v;
-}
-
 // Walks src[0..n) in order on thread 0, one LDS-staged block at a time; the
 // whole workgroup stages. body(stage, base, count) returns true to stop.
 template <uint32_t NT, class Body>
@@ -151,57 +104,6 @@ __device__ __forceinline__ void staged_walk(const float *src, uint32_t n, RL_LDS
         __syncthreads();
         if (*stop) break;
     }
-}
-
-// Where every partial sum of the probabilities is exact: the first j in
-// [lo, hi) with base + p[lo] + ... + p[j] >= target, and that sum in *at; or
-// hi, with the sum of them all in *at. Any order of addition gives these exact
-// sums, so a block scan serves. Whole workgroup.
-template <uint32_t NT>
-__device__ __forceinline__ uint32_t exact_first_reaching(const float *probs, uint32_t lo, uint32_t hi, double base, double target,
-                                         RL_LDS double *red, RL_LDS uint32_t *hit, RL_LDS double *hit_sum,
-                                         double *at, const HotRange &hr) {
-    for (uint32_t b = lo; b < hi; b += NT * CI) {
-        const uint32_t j0 = b + threadIdx.x * CI;
-        float pv[CI];
-        double mine = 0.0;
-#pragma unroll
-        for (uint32_t i = 0; i < CI; ++i) {
-            uint32_t w = hr.word;
-            if (j0 + i < hi && !hr.has(j0 + i)) w = ((const RL_GLB uint32_t *)probs)[j0 + i];
-            pv[i] = j0 + i < hi ? __uint_as_float(w) : 0.0f;
-            mine += (double)pv[i];
-        }
-        if (threadIdx.x == 0) *hit = 0xFFFFFFFFu;
-        double step_total;
-        double c = base + block_exclusive<NT, double>(mine, red, &step_total);
-        uint32_t my_hit = 0xFFFFFFFFu;
-        double my_sum = 0.0;
-#pragma unroll
-        for (uint32_t i = 0; i < CI; ++i) {
-            if (my_hit == 0xFFFFFFFFu && j0 + i < hi) {
-                c += (double)pv[i];
-                if (c >= target) {
-                    my_hit = j0 + i;
-                    my_sum = c;
-                }
-            }
-        }
-        if (my_hit != 0xFFFFFFFFu) atomicMin((uint32_t *)hit, my_hit);
-        __syncthreads();
-        const uint32_t h = *hit;
-        if (h != 0xFFFFFFFFu) {
-            if (my_hit == h) *hit_sum = my_sum;
-            __syncthreads();
-            *at = *hit_sum;
-            __syncthreads();
-            return h;
-        }
-        base += step_total;
-        __syncthreads();
-    }
-    *at = base;
-    return hi;
 }
 
 // What a pass needs of its row.
@@ -384,51 +286,6 @@ __device__ __forceinline__ void digit_prefix(RL_LDS const uint32_t *src, RL_LDS 
         dst[4 * lane + q] = run;
         run += v[q];
     }
-}
-
-// A thread's share of the candidate list's statistics (those kept in LDS
-// beside the segments): p at index j seen by add.
-struct PStats {
-    int emin = 1 << 20;
-    uint32_t bad = 0, count = 0, last_in = 0, first_out = 0xFFFFFFFFu;
-    __device__ __forceinline__ void add(float p, uint32_t j, float min_p) {
-        if (!(p <= 3.40282347e38f)) {
-            bad = 1;  // NaN or +inf
-        } else if (p > 0.0f) {
-            emin = min(emin, f32_exponent(p));
-        }
-        if (p >= min_p) {
-            ++count;
-            last_in = max(last_in, j + 1);
-        } else {
-            first_out = min(first_out, j);
-        }
-    }
-    // Folds the wave's shares into L's (lane 0 adds them with LDS atomics,
-    // after L's were set by stats_reset and a barrier).
-    __device__ __forceinline__ void merge(RL_LDS RestLds *L) {
-        emin = (int)wave_fold_u32((uint32_t)emin, [](uint32_t a, uint32_t b) { return (int)a < (int)b ? a : b; });
-        bad = wave_fold_u32(bad, [](uint32_t a, uint32_t b) { return a | b; });
-        count = wave_sum_u32(count);
-        last_in = wave_fold_u32(last_in, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
-        first_out = wave_fold_u32(first_out, [](uint32_t a, uint32_t b) { return a < b ? a : b; });
-        if (lane_id() == 0) {
-            atomicMin((int *)&L->st_emin, emin);
-            atomicOr((uint32_t *)&L->st_bad, bad);
-            atomicAdd((uint32_t *)&L->st_count, count);
-            atomicMax((uint32_t *)&L->st_last_in, last_in);
-            atomicMin((uint32_t *)&L->st_first_out, first_out);
-        }
-    }
-};
-
-// The list statistics before any merge (one thread).
-__device__ __forceinline__ void stats_reset(RL_LDS RestLds *L) {
-    L->st_emin = 1 << 20;
-    L->st_bad = 0;
-    L->st_count = 0;
-    L->st_last_in = 0;
-    L->st_first_out = 0xFFFFFFFFu;
 }
 
 // Two passes on digits 2 and 3 (keys whose low 16 bits are one value per sign,

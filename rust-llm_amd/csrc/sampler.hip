@@ -36,6 +36,9 @@ constexpr uint32_t MAX_VOCAB = 1u << 21;
 constexpr uint32_t TARGET_WGS = 1024;  // enough workgroups to cover 256 CUs four deep
 constexpr uint32_t FULL_GROUP_MAX = 256;
 constexpr uint32_t CHUNK_SLOTS = 2 * TARGET_WGS;
+constexpr uint32_t SEL_TARGET_WGS = 512;
+constexpr uint32_t SEL_HEAD_WGS = 256;
+static_assert((MAX_VOCAB + SEL_CHUNK_MAX - 1) / SEL_CHUNK_MAX <= MAX_CHUNKS, "the gather's chunks");
 
 enum class Path : uint8_t { Greedy, Stream, Full };
 
@@ -55,6 +58,13 @@ Path plan_row(const rl_sampling &s, uint32_t vocab) {
     if (s.temperature <= 0.0f) return Path::Greedy;
     if (s.top_k >= 1 && s.top_k <= KMAX && s.top_k < vocab) return Path::Stream;
     return Path::Full;
+}
+
+// Whether a full-path row may take the selection path (select_eligible of
+// full_kernels.h, which the kernels decide by).
+bool takes_selection(const rl_sampling &s, uint32_t vocab) {
+    const bool by_k = s.top_k != 0 && s.top_k < vocab;
+    return s.temperature > 0.0f && (by_k || (s.top_p < 1.0f && !(s.min_p > 0.0f)));
 }
 
 uint64_t row_cand_need(const rl_sampling &s, uint32_t vocab) {
@@ -229,6 +239,10 @@ struct rl_sampler_ctx {
     uint64_t *d_surv = nullptr;
     FullRow *d_full_row = nullptr;
     uint32_t *d_full_arrive = nullptr;
+    uint32_t *d_sel_cnt = nullptr, *d_sel_n = nullptr, *d_sel_off = nullptr, *d_sel_fill = nullptr;
+    uint32_t *d_sel_mass = nullptr;
+    double *d_sel_tail = nullptr;
+    uint64_t *d_sel_rec = nullptr;
     uint64_t *d_argmax_part = nullptr;
     uint32_t *d_tp_nan = nullptr;
     double *d_tp_sum = nullptr;
@@ -239,6 +253,7 @@ struct rl_sampler_ctx {
     // Host copy of the plan made by configure.
     uint32_t configured = 0;
     std::vector<uint32_t> stream_rows, full_rows, greedy_rows;  // ascending; capacity max_rows
+    std::vector<uint32_t> select_upto;             // [i]: selection rows among full_rows[0..i]; capacity max_rows
     std::vector<uint64_t> need_upto;               // [r]: candidates rows 0..r can keep; capacity max_rows
     uint64_t cand_need = 0;
     bool any_drawing = false;
@@ -289,6 +304,7 @@ int rl_sampler_create(int device, uint32_t max_rows, uint32_t vocab, uint32_t ma
         c->full_rows.reserve(max_rows);
         c->greedy_rows.reserve(max_rows);
         c->need_upto.reserve(max_rows);
+        c->select_upto.reserve(max_rows);
     } catch (const std::bad_alloc &) {
         delete c;
         return fail(RL_ERR_CAPACITY, "out of host memory");
@@ -315,13 +331,24 @@ int rl_sampler_create(int device, uint32_t max_rows, uint32_t vocab, uint32_t ma
     if (e == hipSuccess) e = c->alloc(&c->d_keyB, fg * V);
     if (e == hipSuccess) e = c->alloc(&c->d_idB, fg * V);
     if (e == hipSuccess) e = c->alloc(&c->d_probs, fg * V);
-    if (e == hipSuccess) e = c->alloc(&c->d_part_max, fg * MAX_CHUNKS);
-    if (e == hipSuccess) e = c->alloc(&c->d_part_am, fg * MAX_CHUNKS);
-    if (e == hipSuccess) e = c->alloc(&c->d_psum, fg * MAX_CHUNKS);
+    if (e == hipSuccess) e = c->alloc(&c->d_part_max, fg * FULL_CHUNKS);
+    if (e == hipSuccess) e = c->alloc(&c->d_part_am, fg * FULL_CHUNKS);
+    if (e == hipSuccess) e = c->alloc(&c->d_psum, fg * FULL_CHUNKS);
     if (e == hipSuccess) e = c->alloc(&c->d_surv, fg * SURV_CAP);
     if (e == hipSuccess) e = c->alloc(&c->d_full_row, fg);
     if (e == hipSuccess) e = c->alloc(&c->d_full_arrive, fg);
     if (e == hipSuccess) e = hipMemset(c->d_full_arrive, 0, fg * sizeof(uint32_t));
+    // The selection path's bins return to zero at the end of every pass.
+    if (e == hipSuccess) e = c->alloc(&c->d_sel_cnt, fg * SEL_BINS);
+    if (e == hipSuccess) e = hipMemset(c->d_sel_cnt, 0, fg * SEL_BINS * sizeof(uint32_t));
+    if (e == hipSuccess) e = c->alloc(&c->d_sel_mass, fg * SEL_BINS);
+    if (e == hipSuccess) e = hipMemset(c->d_sel_mass, 0, fg * SEL_BINS * sizeof(uint32_t));
+    if (e == hipSuccess) e = c->alloc(&c->d_sel_off, fg * (SEL_GROUPS + 1));
+    if (e == hipSuccess) e = c->alloc(&c->d_sel_fill, fg * SEL_GROUPS);
+    if (e == hipSuccess) e = hipMemset(c->d_sel_fill, 0, fg * SEL_GROUPS * sizeof(uint32_t));
+    if (e == hipSuccess) e = c->alloc(&c->d_sel_n, fg * FULL_CHUNKS);
+    if (e == hipSuccess) e = c->alloc(&c->d_sel_tail, fg * FULL_CHUNKS);
+    if (e == hipSuccess) e = c->alloc(&c->d_sel_rec, fg * SEL_GROUPS * 4);
     if (e == hipSuccess) e = c->alloc(&c->d_argmax_part, std::max<size_t>(CHUNK_SLOTS, max_rows));
     if (e == hipSuccess) e = c->alloc(&c->d_tp_nan, std::max<size_t>(CHUNK_SLOTS, max_rows));
     if (e == hipSuccess) e = c->alloc(&c->d_tp_sum, std::max<size_t>(CHUNK_SLOTS, max_rows));
@@ -358,11 +385,16 @@ int rl_sampler_configure(rl_sampler_ctx *ctx, const rl_sampling *settings, uint3
     ctx->full_rows.clear();
     ctx->greedy_rows.clear();
     ctx->need_upto.clear();
+    ctx->select_upto.clear();
     uint64_t need = 0;
     bool drawing = false;
     for (uint32_t r = 0; r < rows; ++r) {
         const Path p = plan_row(settings[r], ctx->vocab);
         (p == Path::Greedy ? ctx->greedy_rows : p == Path::Stream ? ctx->stream_rows : ctx->full_rows).push_back(r);
+        if (p == Path::Full) {
+            const uint32_t before = ctx->select_upto.empty() ? 0u : ctx->select_upto.back();
+            ctx->select_upto.push_back(before + (takes_selection(settings[r], ctx->vocab) ? 1u : 0u));
+        }
         need = std::max(need, row_cand_need(settings[r], ctx->vocab));
         ctx->need_upto.push_back(need);
         drawing = drawing || !(settings[r].temperature <= 0.0f);
@@ -539,16 +571,39 @@ int rl_sampler_sample_rows(rl_sampler_ctx *ctx, const float *logits, uint64_t ro
         const bool consecutive = ctx->full_rows[g0 + ng - 1] - ctx->full_rows[g0] == ng - 1;
         f.rows = consecutive ? nullptr : ctx->d_full_rows + g0;
         f.row0 = ctx->full_rows[g0];
-        f.chunks = std::max(1u, std::min(MAX_CHUNKS, (TARGET_WGS + ng - 1) / ng));
+        // Rows of the group that take the selection path: with any, the pass
+        // counts bins and the gather runs; with no others, few rows are read
+        // in more chunks.
+        const uint32_t nsel = ctx->select_upto[g0 + ng - 1] - (g0 ? ctx->select_upto[g0 - 1] : 0u);
+        const uint32_t most = nsel == ng ? FULL_CHUNKS : MAX_CHUNKS;
+        f.chunks = std::max(1u, std::min(most, (TARGET_WGS + ng - 1) / ng));
         f.chunks = std::min(f.chunks, std::max(1u, vocab / 4096));
-        FullScratch fs{ctx->d_keyA,    ctx->d_idA,     ctx->d_keyB, ctx->d_idB,     ctx->d_probs, ctx->d_part_max,
-                       ctx->d_part_am, ctx->d_psum,    ctx->d_surv, ctx->d_full_row, ctx->d_full_arrive};
-        const dim3 cgrid(f.chunks, ng);
+        // The gather's chunks: two workgroups a CU while rows are few, each of
+        // at least a float4 a thread, at most SEL_CHUNK_MAX elements.
+        uint32_t gchunks = std::max(1u, std::min({FULL_CHUNKS, SEL_TARGET_WGS / ng, vocab / (4 * SEL_THREADS)}));
+        gchunks = std::max(gchunks, (vocab + SEL_CHUNK_MAX - 1) / SEL_CHUNK_MAX);
+        FullScratch fs{ctx->d_keyA,     ctx->d_idA,      ctx->d_keyB,     ctx->d_idB,        ctx->d_probs,
+                       ctx->d_part_max, ctx->d_part_am,  ctx->d_psum,     ctx->d_surv,       ctx->d_full_row,
+                       ctx->d_full_arrive, f.chunks,     gchunks,         ctx->d_sel_cnt,    ctx->d_sel_mass,
+                       ctx->d_sel_off,  ctx->d_sel_fill, ctx->d_sel_n,    ctx->d_sel_tail,   ctx->d_sel_rec};
+        const dim3 cgrid(f.chunks, ng), ggrid(gchunks, ng);
         const size_t pass_lds = k_full_pass_lds_bytes(vocab, f.chunks);
-        if (vec)
-            hipLaunchKernelGGL(k_full_pass<true>, cgrid, dim3(FULL_THREADS), pass_lds, st, f, fs);
-        else
-            hipLaunchKernelGGL(k_full_pass<false>, cgrid, dim3(FULL_THREADS), pass_lds, st, f, fs);
+        if (nsel) {
+            // A row's workgroups share a long head's groups, while rows are few.
+            const uint32_t head_wgs = std::max(1u, std::min(MAX_CHUNKS, SEL_HEAD_WGS / ng));
+            if (vec) {
+                hipLaunchKernelGGL((k_full_pass<true, true>), cgrid, dim3(FULL_THREADS), pass_lds, st, f, fs);
+                hipLaunchKernelGGL(k_full_gather<true>, ggrid, dim3(SEL_THREADS), 0, st, f, fs);
+            } else {
+                hipLaunchKernelGGL((k_full_pass<false, true>), cgrid, dim3(FULL_THREADS), pass_lds, st, f, fs);
+                hipLaunchKernelGGL(k_full_gather<false>, ggrid, dim3(SEL_THREADS), 0, st, f, fs);
+            }
+            hipLaunchKernelGGL(k_full_head, dim3(head_wgs, ng), dim3(SEL_THREADS), 0, st, f, fs);
+        } else if (vec) {
+            hipLaunchKernelGGL((k_full_pass<true, false>), cgrid, dim3(FULL_THREADS), pass_lds, st, f, fs);
+        } else {
+            hipLaunchKernelGGL((k_full_pass<false, false>), cgrid, dim3(FULL_THREADS), pass_lds, st, f, fs);
+        }
         hipLaunchKernelGGL(k_full_rest, dim3(ng), dim3(REST_THREADS), 0, st, f, fs);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return hip_fail(e, "full-path kernels");

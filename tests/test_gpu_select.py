@@ -1,0 +1,148 @@
+"""The selection path on the GPU (top-k above 64, and top-p over the whole
+vocabulary) against the oracle, bit for bit: heads of a few elements, around
+the 4096 that one workgroup finishes, and of many groups; rows it hands to the
+whole-row sort (ties, NaN, a top-p near 1); odd and unaligned rows; rows of it
+beside rows of the other paths in one call; calls repeated on one context."""
+import numpy as np
+import pytest
+
+import rl_sampler as R
+from test_gpu_long_windows import assert_rows_match, run_case
+
+pytestmark = pytest.mark.gpu
+
+
+def logits_of(kind, rng, rows, V):
+    x = rng.normal(0.0, 2.0, (rows, V))
+    if kind == "zipf":
+        x = rng.normal(0.0, 3.0, (rows, V)) - 1.1 * np.log(rng.permutation(V) + 1.0)
+    elif kind == "offset":     # every logit in one octave
+        x += 24.0
+    elif kind == "flat":
+        x *= 0.005
+    elif kind == "bf16":
+        x = (x.astype(np.float32).view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32)
+    elif kind == "masked":     # most ids ruled out
+        x[:, rng.random(V) < 0.9] = -np.inf
+    elif kind == "outlier":    # one logit far above the rest crowds the sort's buckets
+        x[:, V // 3] = 3e4
+    elif kind == "tied":       # one value for all but a few
+        x[:, :] = 1.5
+        x[:, :: 97] = rng.normal(0.0, 1.0, x[:, :: 97].shape)
+    elif kind == "specials":
+        x[0, 5] = np.nan
+        x[1, V - 1] = np.inf
+        x[2, :] = -np.inf
+        x[3, V // 2] = -np.nan
+        x[4, :] = np.nan
+        x[5, :] = -np.inf
+        x[5, 7] = -3.0
+        x[6, :2000] = -np.inf  # the sample of the reference value
+        x[7, :] = 0.0
+        x[7, ::2] = -0.0
+    return x.astype(np.float32)
+
+
+SETTINGS = [
+    R.sampling(0.8, 65, 0.95, 0.0, 1.0, 0, 1),
+    R.sampling(1.0, 100, 1.0, 0.0, 1.3, 64, 2),
+    R.sampling(1.2, 4095, 0.999, 0.0, 1.1, 64, 3),
+    R.sampling(3.0, 4096, 0.9, 0.0, 1.0, 0, 4),
+    R.sampling(2.0, 4097, 1.0, 0.001, 1.0, 0, 5),
+    R.sampling(2.0, 9000, 0.97, 0.0, 0.8, 64, 6),
+    R.sampling(1.0, 100, 0.9, 0.2, 1.0, 0, 7),
+    R.sampling(0.05, 300, 0.95, 0.0, 1.0, 0, 8),       # p far below the sums' exact range
+    R.sampling(0.7, 0, 0.8, 0.0, 1.1, 64, 9),
+    R.sampling(1.0, 0, 0.95, 0.0, 1.0, 0, 10),
+    R.sampling(1.5, 0, 0.99, 0.0, 1.2, 64, 11),
+    R.sampling(0.01, 0, 0.9, 0.0, 1.0, 0, 12),
+    R.sampling(4.0, 0, 0.9, 0.0, 1.0, 0, 13),
+    R.sampling(1.0, 0, 0.99999, 0.0, 1.0, 0, 14),
+    R.sampling(1.0, 0, 0.0, 0.0, 1.0, 0, 15),
+    R.sampling(1.0, 0, 1e-30, 0.0, 1.0, 0, 16),
+]
+
+
+def settings_for(V, rows):
+    out = []
+    for r in range(rows):
+        s = SETTINGS[r % len(SETTINGS)]
+        if s.top_k >= V:
+            s = R.sampling(s.temperature, V - 1, s.top_p, s.min_p, s.repeat_penalty, s.repeat_last_n, s.seed)
+        out.append(s)
+    return out
+
+
+def check(device, label, logits, settings, rng):
+    rows, V = logits.shape
+    win = rng.integers(0, V + 5, (rows, 64)).astype(np.uint32)
+    top = np.argsort(np.nan_to_num(logits, nan=-1e30), axis=1)[:, -24:]
+    win[:, 8:32] = top  # ids the penalty moves
+    wlen = rng.integers(0, 65, rows).astype(np.uint32)
+    u = rng.random(rows).astype(np.float32)
+    u[0] = np.float32(1.0 - 2.0 ** -24)
+    got, want = run_case(device, logits, settings, win, wlen, u, "own", max_window=64)
+    assert_rows_match(label, got, want, settings)
+
+
+@pytest.mark.parametrize("kind", ["normal", "zipf", "offset", "flat", "bf16", "masked", "outlier", "tied", "specials"])
+@pytest.mark.parametrize("V", [4099, 50004])
+def test_heads_match_the_oracle(device, kind, V):
+    print("select", kind, V, flush=True)
+    rng = np.random.default_rng([ord(c) for c in kind] + [V])
+    logits = logits_of(kind, rng, len(SETTINGS), V)
+    check(device, kind, logits, settings_for(V, len(SETTINGS)), rng)
+
+
+@pytest.mark.parametrize("V", [66, 257, 1023, 8193, 151937])
+def test_vocabulary_edges(device, V):
+    print("select vocabulary", V, flush=True)
+    rng = np.random.default_rng(V)
+    rows = 8
+    logits = logits_of("zipf", rng, rows, V)
+    st = settings_for(V, 16)
+    check(device, "V %d top-k" % V, logits, st[:rows], rng)
+    check(device, "V %d top-p" % V, logits, st[8:8 + rows], rng)
+
+
+@pytest.mark.parametrize("rows", [1, 3, 70, 300])
+def test_rows_beside_other_paths(device, rows):
+    print("select mixed", rows, flush=True)
+    rng = np.random.default_rng(rows)
+    V = 9001
+    logits = logits_of("zipf", rng, rows, V)
+    st = settings_for(V, rows)
+    for r in range(rows):
+        if r % 5 == 3:
+            st[r] = R.sampling(1.0, 0, 0.95, 0.05, 1.0, 0, r)     # min-p
+        elif r % 11 == 7:
+            st[r] = R.sampling(0.6, 20, 0.95, 0.0, 1.0, 0, r)     # stream
+        elif r % 13 == 5:
+            st[r] = R.sampling(1.0, 0, 1.0, 0.0, 1.0, 0, r)       # id order
+    check(device, "mixed %d" % rows, logits, st, rng)
+
+
+def test_a_context_is_reused(device):
+    """Bins and counters return to zero: calls over other logits on one
+    context, without candidates, equal the same calls on a new one."""
+    import torch
+    V, rows = 30011, 6
+    st = settings_for(V, 16)[5:11]
+    ctx = R.DeviceSampler(rows, V, max_window=64)
+    ctx.configure(st)
+    for i, kind in enumerate(["zipf", "normal", "specials", "flat", "zipf", "normal"]):
+        rng = np.random.default_rng(100 + i)
+        x = logits_of(kind, rng, max(rows, 8), V)[:rows]
+        u = torch.from_numpy(rng.random(rows).astype(np.float32)).to(device)
+        d = torch.from_numpy(x).to(device)
+        res = []
+        for c in (ctx, None):
+            if c is None:
+                c = R.DeviceSampler(rows, V, max_window=64)
+                c.configure(st)
+            tok = torch.empty(rows, dtype=torch.int32, device=device)
+            kept, used = torch.empty_like(tok), torch.empty(rows, dtype=torch.uint8, device=device)
+            c.sample_rows(d, rows, V, tok, kept, used, uniforms=u)
+            torch.cuda.synchronize()
+            res.append((tok.tolist(), kept.tolist(), used.tolist()))
+        assert res[0] == res[1], (kind, res)
