@@ -321,89 +321,130 @@ __device__ __forceinline__ bool finish_wave(const RowIO &a, uint32_t row, const 
     return true;
 }
 
+constexpr uint32_t DRAW_BLOCK = 32;
+
+// The draw (sample.rs:349-358) over the m terms q[0..m) in LDS: the index of
+// the first whose running f32 sum exceeds u, or m - 1. q is 16-byte aligned and
+// holds zeros from m to the next multiple of DRAW_BLOCK. One wave, every lane
+// alike: the sum is one chain of additions, so the rest is kept off it: the
+// next block's reads are in flight, and only a block's last sum is compared
+// (the sums never fall).
+__device__ __forceinline__ uint32_t draw_walk(RL_LDS const uint32_t *q, uint32_t m, float u) {
+    typedef float vf4 __attribute__((ext_vector_type(4)));
+    vf4 nx[DRAW_BLOCK / 4];
+#pragma unroll
+    for (uint32_t i = 0; i < DRAW_BLOCK / 4; ++i) nx[i] = *(RL_LDS const vf4 *)&q[4 * i];
+    float run = 0.0f;
+    for (uint32_t j = 0; j < m; j += DRAW_BLOCK) {
+        vf4 x[DRAW_BLOCK / 4];
+#pragma unroll
+        for (uint32_t i = 0; i < DRAW_BLOCK / 4; ++i) x[i] = nx[i];
+        const uint32_t jn = j + DRAW_BLOCK < m ? j + DRAW_BLOCK : j;
+#pragma unroll
+        for (uint32_t i = 0; i < DRAW_BLOCK / 4; ++i) nx[i] = *(RL_LDS const vf4 *)&q[jn + 4 * i];
+        float c = run;
+#pragma unroll
+        for (uint32_t i = 0; i < DRAW_BLOCK; ++i) c += x[i / 4][i & 3u];
+        if (c > u) {
+            c = run;
+            uint32_t hit = DRAW_BLOCK;
+#pragma unroll
+            for (uint32_t i = 0; i < DRAW_BLOCK; ++i) {
+                c += x[i / 4][i & 3u];
+                if (hit == DRAW_BLOCK && c > u) hit = i;
+            }
+            return min(j + hit, m - 1);
+        }
+        run = c;
+    }
+    return m - 1;
+}
+
 // The same finish for 64 < c <= FIN_CAP survivors: sv holds their
 // keep_order composites, sorted here by the workgroup (NT threads); sp gets
-// their p; one thread then walks them in order exactly as the reference does
-// (the f64 cut and total, the f32 draw), and the workgroup writes the kept
-// candidates. Every thread returns the same verdict.
+// their p, and room up to the next multiple of DRAW_BLOCK. One wave replays the
+// reference's sums in order (the f64 cut and total, the f32 draw) from LDS
+// reads that run ahead of the additions, and the workgroup writes the kept
+// candidates. Every thread returns the same verdict. A row of 75 survivors
+// among 64 rows of a few makes the call as slow as its finish: one thread
+// walking the list after a sorting network took 18 us, half of the call.
 template <uint32_t NT>
 __device__ __forceinline__ bool finish_block(const RowIO &a, uint32_t row, const rl_sampling &s, float M, uint32_t c,
                                              RL_LDS uint64_t *sv, RL_LDS float *sp, RL_LDS uint32_t *sh,
                                              RL_LDS float *sh_inv, const LdsExpTable &etab, bool by_id,
                                              uint32_t ns_key, double t_lo, double t_hi) {
-    const uint32_t tid = threadIdx.x;
-    uint32_t n2 = 1;
-    while (n2 < c) n2 <<= 1;
-    for (uint32_t i = c + tid; i < n2; i += NT) sv[i] = 0;
-    __syncthreads();
-    lds_bitonic_desc(sv, n2, NT);
+    const uint32_t tid = threadIdx.x, wave = tid / WAVE;
+    const float u = ((const RL_GLB float *)a.uniforms)[row];
+    if (c <= NT) {
+        // A survivor a thread: its place is the number of survivors above it.
+        const uint64_t x = sv[min(tid, c - 1)];
+        uint32_t r = 0;
+#pragma unroll 8
+        for (uint32_t j = 0; j < c; ++j) r += sv[j] > x ? 1u : 0u;
+        __syncthreads();
+        if (tid < c) sv[r] = x;
+        __syncthreads();
+    } else {
+        uint32_t n2 = 1;
+        while (n2 < c) n2 <<= 1;
+        for (uint32_t i = c + tid; i < n2; i += NT) sv[i] = 0;
+        __syncthreads();
+        lds_bitonic_desc(sv, n2, NT);
+    }
     for (uint32_t i = tid; i < c; i += NT) sp[i] = expf_libm_t((key_value(keep_key(sv[i], by_id)) - M) / s.temperature, etab);
+    if (tid == 0) sh[1] = 0;
     __syncthreads();
-    if (tid == 0) {
-        // sh[0]: kept (0 when the row is left to k_full_rest), sh[1]: the drawn index.
+    if (wave == 0) {
+        // sh[0]: kept (0 when the row is left to k_full_rest), sh[1]: a q that is not finite.
+        RL_LDS const uint32_t *pw = (RL_LDS const uint32_t *)sp;
         uint32_t kept = c;
         double total = 0.0;
         bool ok = true;
-        if (!by_id && ns_key != 0 && !(keep_key(sv[c - 1], false) >= ns_key)) ok = false;
-        if (ok && !by_id && !(s.top_p > 0.0f)) {
+        if (by_id) {
+            seq_walk<53>(pw, c, NeverStop(), total);
+        } else if (ns_key != 0 && !(keep_key(sv[c - 1], false) >= ns_key)) {
+            ok = false;
+        } else if (!(s.top_p > 0.0f)) {
             kept = 1;  // sample.rs:315-323
             total = (double)sp[0];
-        } else if (ok && !by_id) {
-            double cum = 0.0;
-            uint32_t j_lo = c, j_hi = c;
-            for (uint32_t j = 0; j < c; ++j) {
-                cum += (double)sp[j];
-                if (j_lo == c && cum >= t_lo) {
-                    j_lo = j;
-                    total = cum;
-                }
-                if (cum >= t_hi) {
-                    j_hi = j;
-                    break;
-                }
+        } else {
+            // The first sum to reach t_lo; the cut is certain when it reaches t_hi too.
+            const uint32_t j = seq_walk<53>(pw, c, [t_lo](double x) { return x >= t_lo; }, total);
+            if (j < c) {
+                ok = total >= t_hi;
+                kept = j + 1;
             }
-            if (j_lo == c) total = cum;                  // no cut among the survivors
-            else if (j_hi != j_lo) ok = false;           // the cut could fall on either side
-            else kept = j_lo + 1;
-        } else if (ok) {
-            for (uint32_t j = 0; j < kept; ++j) total += (double)sp[j];
         }
-        float inv = 0.0f;
-        uint32_t pick = 0;
-        if (ok) {
-            inv = (float)(1.0 / total);
-            float cum = 0.0f;  // the draw, sample.rs:349-358
-            const float u = a.uniforms[row];
-            pick = kept - 1;
-            for (uint32_t j = 0; j < kept; ++j) {
-                const float q = sp[j] * inv;
-                if (!(q <= 3.40282347e38f)) ok = false;
-                cum += q;
-                if (cum > u) {
-                    pick = j;
-                    break;
-                }
-            }
-            for (uint32_t j = pick + 1; ok && j < kept; ++j)
-                if (!(sp[j] * inv <= 3.40282347e38f)) ok = false;
+        if (tid == 0) {
+            sh[0] = ok ? kept : 0u;
+            *sh_inv = (float)(1.0 / total);
         }
-        sh[0] = ok ? kept : 0u;
-        sh[1] = pick;
-        *sh_inv = inv;
     }
     __syncthreads();
     const uint32_t kept = sh[0];
     if (kept == 0) return false;
     const float inv = *sh_inv;
-    if (a.out_ids)
-        for (uint32_t i = tid; i < kept; i += NT) {
-            a.out_ids[(uint64_t)row * a.cand_stride + i] = keep_id(sv[i], by_id);
-            a.out_probs[(uint64_t)row * a.cand_stride + i] = sp[i] * inv;
+    const uint32_t padded = (kept + DRAW_BLOCK - 1) / DRAW_BLOCK * DRAW_BLOCK;
+    for (uint32_t i = tid; i < padded; i += NT) {
+        const float q = i < kept ? sp[i] * inv : 0.0f;
+        if (!(q <= 3.40282347e38f)) sh[1] = 1;
+        sp[i] = q;
+    }
+    __syncthreads();
+    if (sh[1]) return false;
+    if (wave == 0) {
+        // The draw, while the other waves write the candidates.
+        const uint32_t pick = draw_walk((RL_LDS const uint32_t *)sp, kept, u);
+        if (tid == 0) {
+            a.out_token[row] = keep_id(sv[pick], by_id);
+            a.out_kept[row] = kept;
+            a.out_used[row] = 1;
         }
-    if (tid == 0) {
-        a.out_token[row] = keep_id(sv[sh[1]], by_id);
-        a.out_kept[row] = kept;
-        a.out_used[row] = 1;
+    } else if (a.out_ids) {
+        for (uint32_t i = tid - WAVE; i < kept; i += NT - WAVE) {
+            a.out_ids[(uint64_t)row * a.cand_stride + i] = keep_id(sv[i], by_id);
+            a.out_probs[(uint64_t)row * a.cand_stride + i] = sp[i];
+        }
     }
     return true;
 }

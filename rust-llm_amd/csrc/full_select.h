@@ -311,8 +311,6 @@ __device__ __forceinline__ void bucket_sort(const uint64_t (&x)[E], uint32_t n, 
 }
 
 // --------------------------------------------------------- the finish ---
-constexpr uint32_t DRAW_BLOCK = 32;
-
 struct FinishLds {
     uint64_t v[SEL_FIN_CAP];                  // the elements, sorted
     __attribute__((aligned(16))) uint32_t p[SEL_FIN_CAP + DRAW_BLOCK];  // their p, then q (f32 words)
@@ -324,43 +322,6 @@ struct FinishLds {
     uint32_t sh_hit, sh_in, sh_out;
     double sh_at;
 };
-
-// The draw (sample.rs:349-358) over the m terms q[0..m) in LDS: the index of
-// the first whose running f32 sum exceeds u, or m - 1. q is 16-byte aligned and
-// holds zeros from m to the next multiple of DRAW_BLOCK. One wave, every lane
-// alike: the sum is one chain of additions, so the rest is kept off it: the
-// next block's reads are in flight, and only a block's last sum is compared
-// (the sums never fall).
-__device__ __forceinline__ uint32_t draw_walk(RL_LDS const uint32_t *q, uint32_t m, float u) {
-    typedef float vf4 __attribute__((ext_vector_type(4)));
-    vf4 nx[DRAW_BLOCK / 4];
-#pragma unroll
-    for (uint32_t i = 0; i < DRAW_BLOCK / 4; ++i) nx[i] = *(RL_LDS const vf4 *)&q[4 * i];
-    float run = 0.0f;
-    for (uint32_t j = 0; j < m; j += DRAW_BLOCK) {
-        vf4 x[DRAW_BLOCK / 4];
-#pragma unroll
-        for (uint32_t i = 0; i < DRAW_BLOCK / 4; ++i) x[i] = nx[i];
-        const uint32_t jn = j + DRAW_BLOCK < m ? j + DRAW_BLOCK : j;
-#pragma unroll
-        for (uint32_t i = 0; i < DRAW_BLOCK / 4; ++i) nx[i] = *(RL_LDS const vf4 *)&q[jn + 4 * i];
-        float c = run;
-#pragma unroll
-        for (uint32_t i = 0; i < DRAW_BLOCK; ++i) c += x[i / 4][i & 3u];
-        if (c > u) {
-            c = run;
-            uint32_t hit = DRAW_BLOCK;
-#pragma unroll
-            for (uint32_t i = 0; i < DRAW_BLOCK; ++i) {
-                c += x[i / 4][i & 3u];
-                if (hit == DRAW_BLOCK && c > u) hit = i;
-            }
-            return min(j + hit, m - 1);
-        }
-        run = c;
-    }
-    return m - 1;
-}
 
 // The finish of a row of n <= SEL_FIN_CAP collected elements by one
 // workgroup: L->v holds them sorted, tail is the sum of every other p (0 for
