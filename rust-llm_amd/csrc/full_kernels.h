@@ -18,9 +18,12 @@
 // sequential rounding in parallel. Rows with a NaN or infinite p (NaN logits,
 // a NaN temperature, 1 / total overflowing) are walked in order by one thread.
 #pragma once
+#include <type_traits>
+
 #include "minp_bound.h"
 #include "sampler_kernels.h"
 #include "select_bins.h"
+#include "value_bins.h"
 
 namespace rl {
 
@@ -32,6 +35,7 @@ struct FullRow {
     uint32_t count;    // elements in bins 0..thr
     uint32_t groups;   // groups they are sorted in
     uint32_t binned;   // the row was counted into bins (they are cleared by k_full_head)
+    uint32_t values;   // the window its values were counted in (value_bins.h), or 0
 };
 
 // Most chunks of a row on the full path: one lane of a wave each. A launch with
@@ -44,7 +48,7 @@ constexpr uint32_t SURV_CAP = 4096;
 static_assert(FULL_CHUNKS <= WAVE && MAX_CHUNKS <= FULL_CHUNKS, "a wave holds one lane per chunk");
 
 struct FullScratch {
-    uint32_t *keyA, *idA, *keyB, *idB;  // [slot][vocab] k_full_rest: the sort's passes
+    uint32_t *keyA, *idA, *keyB, *idB;  // [slot][vocab] k_full_rest: the sort's passes (keyA: counts first, chunk_counts)
     float *probs;                       // [slot][vocab] k_full_rest: p when the candidates are not returned
     float *part_max;                    // [slot][chunk] k_full_pass: the chunk's maximum
     uint64_t *part_am;                  // [slot][chunk] k_full_pass: candidates listed << 32 | lowest +inf id
@@ -113,6 +117,12 @@ __device__ __forceinline__ bool small_eligible(const rl_sampling &s, uint32_t V)
 // whole vocabulary (with min-p on it tries the min-p path).
 __device__ __forceinline__ bool select_eligible(const rl_sampling &s, uint32_t V) {
     return s.temperature > 0.0f && (full_k(s, V) < V || (s.top_p < 1.0f && !(s.min_p > 0.0f)));
+}
+
+// A value row's counts of each value in a chunk: VAL_BINS / 2 words of two. The
+// tables take the row's keyA (at most vocab / 4096 chunks).
+__device__ __forceinline__ uint32_t *chunk_counts(const FullScratch &f, uint32_t V, uint32_t slot, uint32_t chunk) {
+    return f.keyA + (uint64_t)slot * V + chunk * (VAL_BINS / 2);
 }
 
 // LDS bytes of a chunk's window bitmap: one bit per element of the largest
@@ -468,7 +478,13 @@ __host__ __device__ inline size_t k_full_pass_lds_bytes(uint32_t vocab, uint32_t
 // With SEL (some row of the launch takes the selection path), such rows'
 // elements are also counted into the row's bins, with their mass, for
 // k_full_gather, which takes such rows from there.
-template <bool VEC, bool SEL>
+// With VAL (the call takes no candidates and a chunk's counts fit 16 bits), a
+// row that tries the min-p path with top-p on and that a sample of 64 logits
+// calls nearly flat and on the bf16 grid (half of the sample within min-p's
+// reach of its maximum, so the min-p path would find far more survivors than it
+// finishes) has its values counted instead: each chunk leaves its counts in
+// chunk_counts and lists the elements without a bin, for k_full_rest.
+template <bool VEC, bool SEL, bool VAL>
 __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScratch f) {
     extern __shared__ __align__(16) uint8_t smem[];
     RL_LDS uint32_t *bm = (RL_LDS uint32_t *)smem;  // window ids in this chunk, one bit per element
@@ -482,8 +498,10 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
     __shared__ uint64_t cbuf[PASS_CAND];  // this chunk's candidates, filtered by its maximum at the end
     __shared__ uint32_t sh_cn, sh_cover;
     __shared__ uint32_t red_cnt[FULL_CHUNKS];   // the finisher: each chunk's listed candidates
-    __shared__ uint32_t bin_cnt[SEL ? SEL_BINS : 1];  // the chunk's bins
-    __shared__ uint32_t bin_mass[SEL ? SEL_BINS : 1];
+    // The chunk's bins: a selection row's counts and masses, or its values'.
+    __shared__ uint32_t bins[SEL ? 2 * SEL_BINS : VAL ? VAL_BINS : 1];
+    static_assert(2 * SEL_BINS >= VAL_BINS, "the values' bins fit the selection's");
+    uint32_t *const bin_cnt = bins, *const bin_mass = bins + (SEL ? SEL_BINS : 0);
     const uint32_t slot = blockIdx.y, chunk = blockIdx.x;
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / WAVE;
     const uint32_t row = a.rows ? a.rows[slot] : a.row0 + slot;
@@ -538,6 +556,11 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
 #pragma unroll
         for (uint32_t u = 0; u < PASS_U; ++u) A[u] = pass_load<VEC>(rs, rowp, q0 + u * FULL_THREADS + tid, q0, q1);
     }
+    // Every wave takes the same sample of the row, so that all its chunks
+    // decide alike without hearing of each other; it is waited for with the
+    // step (ahead of the step's loads it cost a min-p call 0.5 us).
+    float smp = 0.0f;
+    if constexpr (VAL) smp = ((const RL_GLB float *)rowp)[min(lane, V - 1)];
     // The row's settings and window length, needed from here on (the
     // barrier keeps the wait for them below the step's loads).
     __builtin_amdgcn_sched_barrier(0);
@@ -593,24 +616,54 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
     const float zthr = uniform_f32((float)(((double)logf(s.min_p) * (1.0 + 0x1p-18) - 1e-3) * 1.4426950408889634));
     // The mass needs a finite c2 and threshold (T not tiny or huge, min_p > 0).
     bool mass = eligible && c2 < 3.0e38f && c2 > 0.0f && zthr > -3.0e38f;
+    uint32_t vlo = 0;       // the window the row's values are counted in, or 0
+    uint32_t hot = 0;       // the bits of a value that is counted in registers, this lane's share:
+    uint32_t hot_n = 0;
+    if (VAL && mass && s.top_p < 1.0f && ballot((__float_as_uint(smp) & 0xFFFFu) != 0) == 0) {
+        const float top = uniform_f32(wave_maxnum_f32(smp)), mag = uniform_f32(wave_maxnum_f32(fabsf(smp)));
+        if (2 * (uint32_t)__popcll(ballot((smp - top) * c2 >= zthr)) >= WAVE && mag < __builtin_inff()) {
+            vlo = val_window(__float_as_uint(mag));
+            // A value that many elements share (a padded or tied part of the
+            // vocabulary) would queue a wave's lanes on one LDS counter: the
+            // commonest of sixteen of the sample's is counted in registers.
+            uint32_t best = 0;
+            for (uint32_t i = 0; i < 16; ++i) {
+                const uint32_t v = read_lane_u32(__float_as_uint(smp), i);
+                const uint32_t n = (uint32_t)__popcll(ballot(__float_as_uint(smp) == v));
+                if (n > best && val_bin(v, vlo) != VAL_NONE) {
+                    best = n;
+                    hot = v;
+                }
+            }
+            if (best == 0) vlo = 0;  // none of them has a bin
+        }
+        if (vlo != 0) {
+            mass = false;
+            for (uint32_t i = tid; i < VAL_BINS; i += FULL_THREADS) bins[i] = 0;
+            __syncthreads();
+        }
+    }
     uint64_t *list = f.surv + (uint64_t)slot * SURV_CAP;
 
     float m_run = -__builtin_inff();  // wave-uniform: the wave's maximum so far
     double S = 0.0;                   // per lane: mass relative to m_run
     uint32_t first_inf = 0xFFFFFFFFu;
     bool nan_seen = false;
-    // The penalised logit of element e of this chunk, re-read from memory
-    // (the candidates' rare path; their row was just read).
+    // The penalised logit of element e of this chunk, from memory (rare paths).
     auto value_at = [&](uint32_t e) {
         float v = ((const RL_GLB float *)rowp)[e];
         if (pen && ((bm[(e - e0) >> 5] >> ((e - e0) & 31)) & 1u)) v = penalize(v, s.repeat_penalty);
         return v;
     };
-    // Appends this lane's candidates (the set bits i of mb; id_of(i) is the
-    // vocabulary id of candidate i) to the chunk's LDS buffer: one LDS atomic
-    // per wave, slots by an exclusive scan of the lanes' counts. A full
-    // buffer sends the row to k_full_rest.
-    auto append = [&](uint64_t mb, auto id_of) {
+    // Appends this lane's candidates (the set bits i < N of mb, of values
+    // val_of(i) and vocabulary ids id_of(i)) to the chunk's LDS buffer: one LDS
+    // atomic per wave, slots by an exclusive scan of the lanes' counts. The
+    // values come from the step's registers, one test an element: read again
+    // from memory, a load after another while a lane held several, they cost
+    // most of the 64-row zipf pass's time. A full buffer sends the row to
+    // k_full_rest.
+    auto append = [&](uint64_t mb, auto n_of, auto val_of, auto id_of) {
+        constexpr uint32_t N = decltype(n_of)::value;
         const uint32_t mine = (uint32_t)__popcll(mb);
         const uint32_t incl = wave_incl_u32(mine);
         const uint32_t wtotal = (uint32_t)__builtin_amdgcn_readlane((int)incl, WAVE - 1);
@@ -619,19 +672,18 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
         base = (uint32_t)__builtin_amdgcn_readlane((int)base, 0);
         if (base + wtotal > PASS_CAND) {
             // The buffer is full: the row leaves the min-p path, and nothing
-            // more is listed (or re-read) for it.
+            // more is listed for it.
             if (lane == 0) sh_cover = 1;
             mass = false;
             return;
         }
         uint32_t at = base + incl - mine;
-        while (mb != 0) {
-            const uint32_t i = (uint32_t)__ffsll((unsigned long long)mb) - 1u;
-            mb &= mb - 1ull;
-            const uint32_t e = id_of(i);
-            cbuf[at++] = composite(total_key(value_at(e)), e);
-        }
+#pragma unroll
+        for (uint32_t i = 0; i < N; ++i)
+            if ((mb >> i) & 1ull) cbuf[at++] = composite(total_key(val_of(i)), id_of(i));
     };
+    const auto of_step = std::integral_constant<uint32_t, 4 * PASS_U>();
+    const auto of_one = std::integral_constant<uint32_t, 1>();
     // Counts element x into its bin (select rows).
     auto count = [&](float x) {
         float edge;
@@ -641,9 +693,66 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
                                (uint32_t)(SEL_MASS_ONE * __builtin_amdgcn_exp2f(-edge * c2)), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_WORKGROUP);
     };
+    // Counts element x's value; false when it has no bin.
+    auto count_value = [&](float x) {
+        const uint32_t v = __float_as_uint(x), d = val_dist(v, vlo);
+        const bool in = d - VAL_FIRST <= VAL_LAST - VAL_FIRST;
+        hot_n += v == hot ? 1u : 0u;
+        uint32_t bin = d + ((v >> 31) * VAL_SPAN);
+        if (!in) bin = val_bin(v, vlo);
+        if (v != hot && bin != VAL_NONE)
+            __hip_atomic_fetch_add((RL_LDS uint32_t *)&bins[bin], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        return bin != VAL_NONE;
+    };
+    // A value row's chunk: its values' counts, the elements without a bin, the
+    // maximum and the lowest +inf.
+    if constexpr (VAL) {
+        if (vlo != 0) {
+            float tmax = -__builtin_inff();
+            for (uint32_t b = q0; b < q1; b += PASS_STEP) {
+                if (b != q0) {
+                    const __amdgpu_buffer_rsrc_t rs = step_rsrc(rowp, b, q1);
+#pragma unroll
+                    for (uint32_t u = 0; u < PASS_U; ++u) A[u] = pass_load<VEC>(rs, rowp, b + u * FULL_THREADS + tid, b, q1);
+                }
+                uint64_t mb = 0;  // elements without a bin: bit 4u + c
+#pragma unroll
+                for (uint32_t u = 0; u < PASS_U; ++u) {
+                    const uint32_t qq = b + u * FULL_THREADS + tid;
+                    if (qq >= q1) continue;
+                    const uint32_t off = 4 * qq - e0;
+                    const uint32_t in = pen ? (bm[off >> 5] >> (off & 31)) & 15u : 0u;
+#pragma unroll
+                    for (uint32_t c = 0; c < 4; ++c) {
+                        if ((in >> c) & 1u) A[u][c] = penalize(A[u][c], s.repeat_penalty);
+                        tmax = fmaxf(tmax, A[u][c]);
+                        if (!count_value(A[u][c])) mb |= 1ull << (4 * u + c);
+                    }
+                }
+                if (ballot(mb != 0) != 0 && sh_cover == 0)
+                    append(mb, of_step, [&](uint32_t i) { return A[i >> 2][i & 3u]; },
+                           [&](uint32_t i) { return 4 * (b + (i >> 2) * FULL_THREADS + tid) + (i & 3u); });
+            }
+            if (chunk == C - 1) {  // the last vocab % 4 elements
+                const uint32_t e = 4 * n4 + tid;
+                const bool ok = e < V;
+                const float x = ok ? value_at(e) : 0.0f;
+                if (ok) tmax = fmaxf(tmax, x);
+                const uint64_t mb = ok && !count_value(x) ? 1ull : 0ull;
+                if (ballot(mb != 0) != 0 && sh_cover == 0)
+                    append(mb, of_one, [&](uint32_t) { return x; }, [&](uint32_t) { return e; });
+            }
+            m_run = uniform_f32(wave_maxnum_f32(tmax));
+            if (m_run == __builtin_inff())  // this wave's first +inf (among others'; the row takes the lowest)
+                for (uint32_t e = e1 - 1 - lane; e + 1 > e0 && e < e1; e -= WAVE)
+                    if (value_at(e) == __builtin_inff()) first_inf = e;
+            hot_n = wave_sum_u32(hot_n);
+            if (lane == 0) atomicAdd(&bins[val_bin(hot, vlo)], hot_n);
+        }
+    }
     // A step's PASS_U float4 per thread are all in flight at once (a chunk
     // of the 64-row workload is one step); the penalty is applied in place.
-    for (uint32_t b = q0; b < q1; b += PASS_STEP) {
+    for (uint32_t b = q0; b < q1 && !(VAL && vlo != 0); b += PASS_STEP) {
         if (b != q0) {
             const __amdgpu_buffer_rsrc_t rs = step_rsrc(rowp, b, q1);
 #pragma unroll
@@ -729,7 +838,8 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
                     for (uint32_t c = 0; c < 4; ++c)
                         if (ok && (A[u][c] - m_run) * c2 >= zthr) mb |= 1ull << (4 * u + c);
                 }
-                append(mb, [&](uint32_t i) { return 4 * (b + (i >> 2) * FULL_THREADS + tid) + (i & 3u); });
+                append(mb, of_step, [&](uint32_t i) { return A[i >> 2][i & 3u]; },
+                       [&](uint32_t i) { return 4 * (b + (i >> 2) * FULL_THREADS + tid) + (i & 3u); });
             }
         } else if (eligible && m_run == -__builtin_inff()) {
             // Nothing finite so far: no mass, but a NaN must still send the
@@ -741,7 +851,7 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
                     if (b + u * FULL_THREADS + tid < q1 && A[u][c] != A[u][c]) nan_seen = true;
         }
     }
-    if (chunk == C - 1) {  // the last vocab % 4 elements, one per thread (at most 3)
+    if (chunk == C - 1 && !(VAL && vlo != 0)) {  // the last vocab % 4 elements, one per thread (at most 3)
         const uint32_t e = 4 * n4 + tid;
         float xe = -__builtin_inff();
         const bool ok = e < V;
@@ -764,7 +874,7 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
             const float z = (xe - m_run) * c2;
             if (ok) S += (double)__builtin_amdgcn_exp2f(z);
             const uint64_t mb = (ok && z >= zthr) ? 1ull : 0ull;
-            if (ballot(mb != 0) != 0) append(mb, [&](uint32_t) { return e; });
+            if (ballot(mb != 0) != 0) append(mb, of_one, [&](uint32_t) { return xe; }, [&](uint32_t) { return e; });
         } else if (eligible && ok && xe != xe) {
             nan_seen = true;
         }
@@ -792,7 +902,7 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
     // count goes with the chunk's record; LIST_OVER marks a region too small.
     const uint32_t region = SURV_CAP / C;
     uint32_t nkeep = 0;
-    if (eligible && Mc > -__builtin_inff() && Mc < __builtin_inff() && sh_cover == 0) {
+    if (eligible && (Mc > -__builtin_inff() || (VAL && vlo != 0)) && Mc < __builtin_inff() && sh_cover == 0) {
         const uint32_t n = min(sh_cn, PASS_CAND);
         uint32_t mine = 0;  // this wave's kept candidates, its slice of the buffer
         const uint32_t per = (n + FULL_WAVES - 1) / FULL_WAVES;
@@ -800,7 +910,7 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
         for (uint32_t b = lo; b < hi; b += WAVE) {
             const uint32_t i = b + lane;
             const uint64_t cc = i < hi ? cbuf[i] : 0ull;
-            mine += (uint32_t)__popcll(ballot(i < hi && (key_value(comp_key(cc)) - Mc) * c2 >= zthr));
+            mine += (uint32_t)__popcll(ballot(i < hi && ((VAL && vlo != 0) || (key_value(comp_key(cc)) - Mc) * c2 >= zthr)));
         }
         if (lane == 0) red_f[wave] = mine;
         __syncthreads();
@@ -814,7 +924,7 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
             for (uint32_t b = lo; b < hi; b += WAVE) {
                 const uint32_t i = b + lane;
                 const uint64_t cc = i < hi ? cbuf[i] : 0ull;
-                const bool keep = i < hi && (key_value(comp_key(cc)) - Mc) * c2 >= zthr;
+                const bool keep = i < hi && ((VAL && vlo != 0) || (key_value(comp_key(cc)) - Mc) * c2 >= zthr);
                 const uint64_t mk = ballot(keep);
                 if (keep) __hip_atomic_store(dst + at + lanes_below(mk), cc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 at += (uint32_t)__popcll(mk);
@@ -862,6 +972,17 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
             if (chunk == 0 && tid == 0) f.row[slot].R = ref;
             return;
         }
+    }
+    if (VAL && vlo != 0) {
+        uint32_t *tab_c = chunk_counts(f, V, slot, chunk);
+        for (uint32_t i = tid; i < VAL_BINS / 2; i += FULL_THREADS) tab_c[i] = bins[2 * i] | (bins[2 * i + 1] << 16);
+        if (chunk == 0 && tid == 0) {
+            FullRow st{};
+            st.thr = SEL_NONE;
+            st.values = vlo;
+            f.row[slot] = st;
+        }
+        return;
     }
     __builtin_amdgcn_s_waitcnt(WAITCNT_VM0);  // this wave's stores have completed
     __syncthreads();                          // and every other wave's

@@ -15,7 +15,7 @@
 // pick). A row the pass finished exits at once, so a call whose rows all
 // finished in the pass costs one empty launch here.
 #pragma once
-#include "full_head.h"
+#include "full_values.h"
 
 namespace rl {
 
@@ -589,10 +589,13 @@ __device__ __forceinline__ uint32_t stat_shift(uint32_t k) {
 
 // grid (slots), REST_THREADS: the rows k_full_pass left (done == 0).
 __global__ __launch_bounds__(REST_THREADS) void k_full_rest(RowIO a, FullScratch f) {
-    __shared__ RestLds L_;
-    RL_LDS RestLds *L = (RL_LDS RestLds *)&L_;
+    __shared__ union {
+        RestLds rest;
+        ValLds val;
+    } L_;
+    RL_LDS RestLds *L = (RL_LDS RestLds *)&L_.rest;
     const uint32_t slot = blockIdx.x;
-    const FullRow st = f.row[slot];
+    FullRow st = f.row[slot];
     if (st.done) return;
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / WAVE;
     const uint32_t row = a.rows ? a.rows[slot] : a.row0 + slot;
@@ -600,6 +603,10 @@ __global__ __launch_bounds__(REST_THREADS) void k_full_rest(RowIO a, FullScratch
     const uint32_t V = a.vocab;
     const uint32_t k = full_k(s, V);
     const uint32_t wl = window_len(a, row);
+    if (st.values != 0) {
+        if (finish_values(a, f, slot, row, s, st.values, wl, (RL_LDS ValLds *)&L_.val, &st.M)) return;
+        __syncthreads();  // its LDS is free
+    }
     const RestRow r{a.logits + (uint64_t)row * a.stride,
                     wl > 0 ? a.windows + (uint64_t)row * a.wstride : nullptr,
                     V,

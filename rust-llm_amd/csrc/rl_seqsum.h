@@ -267,6 +267,28 @@ RL_HD inline void run_add(StepRun &r, uint32_t xb, double scale) {
     }
 }
 
+// Appends n >= 1 equal terms. Without a tie each adds the same steps. With one
+// the first term's step depends on the parity before it, as in run_add, and
+// leaves the significand even, so that every later one adds q rounded to even.
+RL_HD inline void run_add_equal(StepRun &r, uint32_t xb, uint32_t n, double scale) {
+    bool t;
+    const double q = step_of(f32_from_bits(xb), scale, &t);
+    if (!t) {
+        r.base += q * (double)n;
+        return;
+    }
+    const uint32_t pq = parity_of(q);
+    if (!r.tie) {
+        r.tie = 1;
+        r.c = parity_of(r.base) ^ pq;
+        r.base += q;
+    } else {
+        r.base += q + (double)(parity_of(r.base - r.mark) ^ pq);
+    }
+    r.base += (q + (double)pq) * (double)(n - 1);
+    r.mark = r.base;
+}
+
 // The run's par: the parity it leaves, relative to the entering one without a
 // tie (p ^ par) and absolute with one.
 RL_HD inline uint32_t run_par(const StepRun &r) { return r.tie ? parity_of(r.base - r.mark) : parity_of(r.base); }
@@ -312,8 +334,8 @@ RL_HD inline bool seg_multiple(const SumSeg &g, int gx) {
 
 // Adds `count` equal terms x (bits xb: finite, >= 0) in order to the running
 // sum s (a P-bit value >= 0, pred(s) false), one segment of the sum at a time.
-// On the grid of s's segment the first term adds map_inc(t, parity) steps and
-// every later one t.i0: a term that is not an exact tie adds the same steps
+// On the grid of s's segment the first term adds `first` steps and every
+// later one `rest`: a term that is not an exact tie adds the same steps
 // from either parity, and a tie leaves the significand even. So the partial
 // sums inside the segment are n + first + (j - 1) * rest for the j-th term, up
 // to the term whose sum would reach the segment's end, which is added with the
@@ -334,34 +356,37 @@ RL_HD inline uint32_t equal_run_walk(double &s, uint32_t xb, uint32_t count, Pre
             ++done;
             continue;
         }
-        const SumSeg g = seg_of<P>(s);
-        const TermMap t = map_of(xb, g.uexp);
-        const uint64_t first = map_inc(t, (uint32_t)(g.n & 1u)), rest = t.i0;
-        const uint64_t left = count - done;
+        const SumSegF g = segf_of<P>(s);
+        bool tie;
+        const double q = step_of(x, mul_pow2(1.0, -g.uexp), &tie);
+        const uint32_t pq = parity_of(q);
+        const double first = tie ? q + (double)(parity_of(g.n) ^ pq) : q, rest = tie ? q + (double)pq : q;
+        const double left = (double)(count - done);
         // K: the terms whose sums stay below the segment's end (at most left).
-        uint64_t K;
-        if (g.n + first >= g.lim) {
-            K = 0;
-        } else if (rest == 0) {
+        // Counts are exact below 2^53; one that is not reads as past the end.
+        double K = 0.0;
+        if (g.n + first < g.lim) {
+            const double a = g.lim - g.n - first;  // K = ceil(a / rest): the j with (j - 1) rest < a
             K = left;
-        } else {
-            const uint64_t a = g.lim - g.n - first;  // the first j with sum >= lim is 1 + ceil(a / rest)
-            const uint64_t jl = 1 + (a + rest - 1) / rest;
-            K = jl - 1 < left ? jl - 1 : left;
+            if (rest * left >= a) {  // so a / rest <= left, up to a rounding
+                K = __builtin_ceil(a / rest);
+                if (K * rest < a) K += 1.0;  // a quotient rounded down to a whole number
+                K = K < left ? K : left;
+            }
         }
-        if (K > 0) {
-            auto sum_at = [&](uint64_t j) { return scaled(g.n + first + (j - 1) * rest, g.uexp); };
+        if (K > 0.0) {
+            auto sum_at = [&](double j) { return mul_pow2(g.n + first + (j - 1.0) * rest, g.uexp); };
             if (pred(sum_at(K))) {
-                uint64_t lo = 1, hi = K;  // the first j in [1, K] meeting pred
+                uint32_t lo = 1, hi = (uint32_t)K;  // the first j in [1, K] meeting pred
                 while (lo < hi) {
-                    const uint64_t mid = lo + (hi - lo) / 2;
-                    if (pred(sum_at(mid)))
+                    const uint32_t mid = lo + (hi - lo) / 2;
+                    if (pred(sum_at((double)mid)))
                         hi = mid;
                     else
                         lo = mid + 1;
                 }
-                s = sum_at(lo);
-                return done + (uint32_t)(lo - 1);
+                s = sum_at((double)lo);
+                return done + (lo - 1);
             }
             s = sum_at(K);
             done += (uint32_t)K;

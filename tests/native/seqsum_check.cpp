@@ -476,10 +476,40 @@ static void run_all(int &cases) {
     }
 }
 
+// run_add_equal(n equal terms) against n run_adds, after a run of other terms:
+// ties, multiples of the step, terms below half a step and plain ones.
+static void check_add_equal(int &cases) {
+    for (int rep = 0; rep < 20000; ++rep) {
+        const int uexp = -(int)(rnd() % 40) - 10;
+        const double scale = ldexp(1.0, -uexp);
+        auto term = [&]() {
+            switch (rnd() % 4) {
+            case 0: return fbits((float)ldexp((double)(2 * (rnd() % 64) + 1), uexp - 1));
+            case 1: return fbits((float)ldexp((double)(rnd() % 4096), uexp));
+            case 2: return fbits((float)ldexp(unit(), uexp - 2));
+            default: return fbits((float)ldexp(unit(), uexp + (int)(rnd() % 20)));
+            }
+        };
+        StepRun a = run_identity();
+        for (uint32_t i = rnd() % 4; i > 0; --i) run_add(a, term(), scale);
+        StepRun b = a;
+        const uint32_t x = term(), n = 1 + (uint32_t)(rnd() % (rep % 50 == 0 ? 3000 : 9));
+        for (uint32_t i = 0; i < n; ++i) run_add(a, x, scale);
+        run_add_equal(b, x, n, scale);
+        const bool same = a.base == b.base && a.tie == b.tie && run_par(a) == run_par(b) && (!a.tie || a.c == b.c);
+        if (!same) {
+            ++failures;
+            printf("FAIL equal terms: rep %d n %u\n", rep, n);
+        }
+        ++cases;
+    }
+}
+
 int main() {
     int cases = 0;
     check_assoc();
     check_runs();
+    check_add_equal(cases);
     run_all<24>(cases);
     run_all<53>(cases);
     check_equal_runs<24>(cases);
