@@ -31,8 +31,8 @@ typedef struct rl_head rl_head;
 /* Uploads a Q6_K weight tensor of `rows` rows of `k` values (ggml layout: each
  * row is ceil(k/256) blocks of 210 bytes, `ql[128] qh[64] scales[16] d:f16`;
  * q6k_bytes must be rows * ceil(k/256) * 210) from HOST memory, repacks it on
- * the device into the layout the head kernel streams (same byte count), and
- * sizes the activation scratch for up to `max_batch` rows per call. Replaces
+ * the device into the layout the head kernel streams (same byte count; the
+ * uploaded form stays beside it for rl_head_embed_rows), and sizes the activation scratch for up to `max_batch` rows per call. Replaces
  * the memory-mapped tensor view the reference's head reads (`model.token_embd`,
  * forward.rs:934; TensorView, crates/llm-core/src/gguf.rs:190-197).
  * Synchronous. */

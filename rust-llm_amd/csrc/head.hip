@@ -20,12 +20,14 @@ struct rl_head {
     uint4 *wq = nullptr;
     uint32_t *ws = nullptr;
     uint16_t *wd = nullptr;
+    uint8_t *q6k = nullptr; // the tensor as uploaded, for the lookup
     float *ad = nullptr;    // activation scales [tcap][nb]
     uint4 *af = nullptr;    // activation fragments [tcap / 16][nb][HEAD_FRAG_UINT4]
     ~rl_head() {
         (void)hipFree(wq);
         (void)hipFree(ws);
         (void)hipFree(wd);
+        (void)hipFree(q6k);
         (void)hipFree(ad);
         (void)hipFree(af);
     }
@@ -101,17 +103,15 @@ int rl_head_create(int device, uint32_t k, uint32_t rows, uint32_t max_batch, co
     // discarded; start them at zero.
     if (e == hipSuccess) e = hipMemset(h->ad, 0, (uint64_t)h->tcap * nb * sizeof(float));
     if (e == hipSuccess) e = hipMemset(h->af, 0, (uint64_t)(h->tcap / HEAD_NTILE) * nb * HEAD_FRAG_UINT4 * sizeof(uint4));
-    uint8_t *staging = nullptr;
-    if (e == hipSuccess) e = hipMalloc(&staging, q6k_bytes);
-    if (e == hipSuccess) e = hipMemcpy(staging, q6k, q6k_bytes, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMalloc(&h->q6k, q6k_bytes);
+    if (e == hipSuccess) e = hipMemcpy(h->q6k, q6k, q6k_bytes, hipMemcpyHostToDevice);
     if (e == hipSuccess) {
         const uint64_t threads = bgt * 64;
-        hipLaunchKernelGGL(k_q6k_repack, dim3((uint32_t)((threads + 255) / 256)), dim3(256), 0, 0, staging, rows,
+        hipLaunchKernelGGL(k_q6k_repack, dim3((uint32_t)((threads + 255) / 256)), dim3(256), 0, 0, h->q6k, rows,
                            nb, h->groups, h->wq, h->ws, h->wd);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipDeviceSynchronize();
-    if (staging) (void)hipFree(staging);
     if (e != hipSuccess) {
         delete h;
         return hip_fail(e, "rl_head_create");
@@ -150,13 +150,15 @@ int rl_head_embed_rows(rl_head *h, const uint32_t *tokens, uint32_t t, float *ou
     if (t == 0) return RL_OK;
     if (!tokens || !out) return fail(RL_ERR_ARGUMENT, "tokens and out must be device pointers");
     if (row_stride < h->k) return fail(RL_ERR_ARGUMENT, "row_stride below k");
-    const uint64_t threads = (uint64_t)t * h->nb * 16;
-    const uint64_t blocks = (threads + EMBED_THREADS - 1) / EMBED_THREADS;
-    if (blocks > 0xFFFFFFFFull) return fail(RL_ERR_CAPACITY, "too many tokens for one launch");
+    if ((uint64_t)t * h->nb > 0xFFFFFFFFull * 16) return fail(RL_ERR_CAPACITY, "too many tokens for one launch");
     DeviceGuard g(h->device);
     if (!g.ok) return fail(RL_ERR_DEVICE, "cannot select the head's device");
-    hipLaunchKernelGGL(k_embed_rows, dim3((uint32_t)blocks), dim3(EMBED_THREADS), 0, static_cast<hipStream_t>(stream),
-                       h->wq, h->ws, h->wd, tokens, t, h->k, h->nb, h->rows, h->groups, out, row_stride);
+    // A launch takes 2^32 threads along an axis: 2^24 tokens of a workgroup each, half of that here.
+    constexpr uint32_t PER = 1u << 23, PER_WG = EMBED_THREADS / 64;
+    for (uint32_t t0 = 0; t0 < t; t0 += std::min(PER, t - t0))
+        hipLaunchKernelGGL(k_embed_rows, dim3(std::min(PER, t - t0), std::min((h->nb + PER_WG - 1) / PER_WG, 65535u)),
+                           dim3(EMBED_THREADS), 0, static_cast<hipStream_t>(stream), h->q6k, tokens + t0, h->k, h->nb,
+                           h->rows, out + (uint64_t)t0 * row_stride, row_stride);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? RL_OK : hip_fail(e, "rl_head_embed_rows launch");
 }

@@ -650,67 +650,63 @@ void k_head_dot(const uint4 *__restrict__ wq, const uint32_t *__restrict__ ws, c
 // ------------------------------------------------------------ embedding lookup
 
 // The reference's embedding lookup (forward.rs:1127-1138), dequantize_row's
-// Q6_K arm (quant.rs:177-203), from the repacked tensor: value i of a row is
-// d * (float)(s * (q - 32)), the integer product exact and one f32 multiply,
-// as the reference forms it. One thread per (token, block, quarter h, step
-// pair p): the row's 16 values 64 h + 16 p .. + 15 of the block, all of
-// sub-block 4 h + p, from words 3p .. 3p+2 of lane 16 h + m's quant chunks (the
-// packing above). A token at or past `rows` gives a row of NaN: the reference
-// asserts (forward.rs:1130-1134), which a kernel cannot.
+// Q6_K arm (quant.rs:177-203): value i of a row is d * (float)(s * (q - 32)),
+// the integer product exact and one f32 multiply, as the reference forms it.
+// It reads the tensor as it was uploaded, a row's blocks side by side: in the
+// matrix-core layout a block lies in 15 cache lines shared with 15 other rows
+// (9.3 times the bytes used were read). 2048 tokens of 2560: 14.9 -> 7.2 us,
+// against about 4 for the bytes used; the launch is most of the rest. One wave per (token, block): lane j writes values 4 j .. 4 j +
+// 3 (a wave 1 KiB in one store) from four bytes of ql, four of qh, the
+// sub-block's scale and d. A token at or past `rows` gives a row of NaN: the
+// reference asserts (forward.rs:1130-1134), which a kernel cannot.
 constexpr int EMBED_THREADS = 256;
 
-__global__ __launch_bounds__(EMBED_THREADS) void k_embed_rows(const uint4 *__restrict__ wq,
-                                                              const uint32_t *__restrict__ ws,
-                                                              const uint16_t *__restrict__ wd,
-                                                              const uint32_t *__restrict__ tokens, uint32_t t,
-                                                              uint32_t k, uint32_t nb, uint32_t rows, uint32_t groups,
-                                                              float *__restrict__ out, uint64_t out_stride) {
-    const uint64_t idx = (uint64_t)blockIdx.x * EMBED_THREADS + threadIdx.x;
-    if (idx >= (uint64_t)t * nb * 16) return;
-    const uint32_t p = (uint32_t)(idx & 3), h = (uint32_t)((idx >> 2) & 3);
-    const uint64_t tb = idx >> 4;
-    const uint32_t ib = (uint32_t)(tb % nb), ti = (uint32_t)(tb / nb);
-    const uint32_t k0 = ib * QK + 64 * h + 16 * p;
-    if (k0 >= k) return;
-    const uint32_t n = k - k0 < 16 ? k - k0 : 16;
-    float *o = out + (uint64_t)ti * out_stride + k0;
-    const uint32_t tok = tokens[ti];
-    float v[16];
-    if (tok >= rows) {
+// The four bytes at p (2-byte aligned, with four readable bytes after them,
+// in a buffer that starts 4-byte aligned).
+__device__ __forceinline__ uint32_t embed_word(const uint8_t *p) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(p);
+    const uint2 w = *reinterpret_cast<const uint2 *>(at & ~(uintptr_t)3);
+    return __builtin_amdgcn_alignbyte(w.y, w.x, (uint32_t)at & 3u);
+}
+
+// grid (tokens, nb / 4 rounded up, or fewer)
+__global__ __launch_bounds__(EMBED_THREADS) void k_embed_rows(const uint8_t *__restrict__ q6k,
+                                                              const uint32_t *__restrict__ tokens, uint32_t k,
+                                                              uint32_t nb, uint32_t rows, float *__restrict__ out,
+                                                              uint64_t out_stride) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t ti = blockIdx.x, tok = tokens[ti];
+    for (uint32_t ib = blockIdx.y * (EMBED_THREADS / 64) + threadIdx.x / 64; ib < nb;
+         ib += gridDim.y * (EMBED_THREADS / 64)) {
+        const uint32_t k0 = ib * QK + 4 * lane;
+        if (k0 >= k) return;
+        const uint32_t n = k - k0 < 4 ? k - k0 : 4;
+        float *o = out + (uint64_t)ti * out_stride + k0;
+        float v[4];
+        if (tok >= rows) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = __builtin_nanf("");
-    } else {
-        const uint32_t g = tok / HEAD_GROUP, tw = (tok / HEAD_TILE) % HEAD_TILES, m = tok % HEAD_TILE;
-        const uint64_t bgt = ((uint64_t)ib * groups + g) * HEAD_TILES + tw;
-        const uint32_t lane = 16 * h + m;
-        const uint32_t *q = reinterpret_cast<const uint32_t *>(wq + bgt * HEAD_QCH * 64 + lane);
-        uint32_t pw[3];
+            for (int i = 0; i < 4; ++i) v[i] = __builtin_nanf("");
+        } else {
+            // Values 4 lane .. of half hf: quarter qd of its 128, from position l.
+            const uint8_t *blk = q6k + ((uint64_t)tok * nb + ib) * Q6K_BLOCK_BYTES;
+            const uint32_t hf = lane / 32, qd = lane / 8 & 3u, l = 4 * (lane & 7u);
+            const uint32_t ql = embed_word(blk + 64 * hf + 32 * (qd & 1u) + l) >> (4 * (qd >> 1));
+            const uint32_t qh = embed_word(blk + 128 + 32 * hf + l) >> (2 * qd);
+            const int s = (int)(int8_t)blk[192 + lane / 4];
+            const float d = __half2float(__ushort_as_half(*reinterpret_cast<const uint16_t *>(blk + 208)));
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const uint32_t wi = 3 * p + j;
-            pw[j] = q[(wi / 4) * 64 * 4 + wi % 4];
+            for (int i = 0; i < 4; ++i) {
+                const int q = (int)((ql >> (8 * i) & 15u) | (qh >> (8 * i) & 3u) << 4);
+                v[i] = d * (float)(s * (q - 32));
+            }
         }
-        const int s = (int)(int8_t)(ws[bgt * 64 + lane] >> (8 * p));
-        const float d = __half2float(__ushort_as_half(wd[bgt * HEAD_TILE + m]));
+        if (n == 4 && (reinterpret_cast<uintptr_t>(o) & 15) == 0) {
+            *reinterpret_cast<float4 *>(o) = make_float4(v[0], v[1], v[2], v[3]);
+        } else {
 #pragma unroll
-        for (int x = 0; x < 2; ++x) {
-            const uint32_t a = pw[0] >> (16 * x), b = pw[1] >> (16 * x), c = pw[2] >> (16 * x);
-            const uint32_t u[8] = {a & 63, (a >> 6) & 63, b & 63, (b >> 6) & 63,
-                                   c & 63, (c >> 6) & 63, ((a >> 12) & 15) | ((c >> 12) & 3) << 4,
-                                   ((b >> 12) & 15) | ((c >> 14) & 3) << 4};
-            // u[j] is value 2 j + x of the sixteen.
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[2 * j + x] = d * (float)(s * ((int)u[j] - 32));
+            for (int i = 0; i < 4; ++i)
+                if ((uint32_t)i < n) o[i] = v[i];
         }
-    }
-    if (n == 16 && (reinterpret_cast<uintptr_t>(o) & 15) == 0) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            reinterpret_cast<float4 *>(o)[j] = make_float4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-            if ((uint32_t)i < n) o[i] = v[i];
     }
 }
 
