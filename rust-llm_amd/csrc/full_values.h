@@ -12,10 +12,9 @@
 // counts and one read of its chunk.
 //
 // What bounds it: one workgroup's chain of dependent steps, with little for its
-// other CUs to take over (256 x 151936, 40 % of a row tied: tables 2 us, runs 5,
-// p 4, cut and total 4, draw 21, the drawn id 7). Sorting these rows took 364 us
-// in k_full_rest after a pass of 32; counting takes 61 after a pass of 41 (its
-// LDS atomics), and the call 385 -> 100 us.
+// other CUs to take over. Sorting these rows (256 x 151936, 40 % of a row tied)
+// took 364 us in k_full_rest after a pass of 32; counting takes 54 after a pass
+// of 41 (its LDS atomics), and the call 385 -> 93 us.
 #pragma once
 #include "full_head.h"
 
@@ -27,9 +26,6 @@ constexpr uint32_t VAL_PER = VAL_RUNS / SEL_THREADS;  // runs a thread
 static_assert(VAL_PER * SEL_THREADS == VAL_RUNS && VAL_BINS == 4 * SEL_THREADS, "the runs over the threads");
 constexpr uint32_t VAL_BLOCK = 16 * WAVE;           // elements of a wave's step through a chunk
 constexpr uint32_t VAL_BLOCKS = 65536 / VAL_BLOCK;
-constexpr uint32_t RUN_HEAD = 48;                   // runs that run_walk adds one by one
-constexpr uint32_t RUN_SHORT = 24;                  // terms that it adds one by one
-static_assert(RUN_HEAD <= WAVE, "a run a lane");
 
 struct ValLds {
     uint64_t exc[VAL_EXC];         // the elements without a bin, sorted
@@ -44,48 +40,25 @@ struct ValLds {
     uint32_t red_u[SEL_WAVES];
     int st_emin;
     uint32_t st_bad, st_count, st_last_in, st_first_out;
-    uint32_t sh_hit, sh_m, sh_pick, sh_run, sh_off, sh_chunk, sh_nth;
+    uint32_t sh_hit, sh_m, sh_run, sh_off, sh_chunk, sh_nth;
     double sh_at;
 };
 
 // One wave adds the R runs of equal terms (n[r] terms with the bits term[r]) to
-// the running sum s (a P-bit value >= 0) in order, every lane alike. Lane l
-// counts the steps of runs pos + l WK .. on the grid of s's segment
-// (run_add_equal), ties resolved as in wave_walk; the first lane whose runs
-// leave the segment or meet pred goes through them one by one, and the run that
-// does so is crossed in closed form (equal_run_walk). Returns the first term
-// whose partial sum meets pred (its place among all terms), with that sum in s,
-// or 0xFFFFFFFF with the total in s.
-template <int P, uint32_t WK, class Pred>
+// a running sum from 0 in order, every lane alike, in f64 (run_walk) or, for
+// the draw, in f32 (run_draw: term[0] >= 2^-60, sums below 2^60, a run a lane).
+// Lane l counts the steps of runs pos + l WK .. on the grid of the sum's segment, ties
+// resolved as in wave_walk; the first lane whose runs leave the segment or meet
+// pred goes through them one by one, and the run that does so is crossed in
+// closed form. Returns the first term whose partial sum meets pred (its place
+// among all terms), with that sum in s, or 0xFFFFFFFF with the total in s.
+template <uint32_t WK, class Pred>
 __device__ __forceinline__ uint32_t run_walk(RL_LDS const uint32_t *term, RL_LDS const uint32_t *n, uint32_t R,
                                              Pred pred, double &s) {
+    constexpr int P = 53;
     const uint32_t lane = lane_id();
     uint32_t before = 0;  // terms added so far
-    uint32_t pos = 0;
-    // One run crossed: its few terms one by one, or in closed form. Returns
-    // whether pred was met (then *at is the term).
-    auto cross = [&](uint32_t xb, uint32_t cnt, uint32_t *at) {
-        uint32_t j = cnt;
-        typedef typename std::conditional<P == 24, float, double>::type acc_t;
-        acc_t run = (acc_t)s;  // a P-bit value: exact
-        if (cnt <= RUN_SHORT)
-            for (uint32_t i = 0; i < cnt; ++i) run += (acc_t)__uint_as_float(xb);
-        if (cnt > RUN_SHORT || pred((double)run)) j = equal_run_walk<P>(s, xb, cnt, pred);
-        else s = (double)run;
-        *at = before + j;
-        before += cnt;
-        return j < cnt;
-    };
-    // The first runs, which take the sum through a binade each or nearly, one
-    // by one.
-    {
-        const uint32_t x = lane < R ? term[lane] : 0u, c = lane < R ? n[lane] : 0u;
-        for (; pos < min(R, RUN_HEAD); ++pos) {
-            uint32_t at;
-            if (cross(read_lane_u32(x, pos), read_lane_u32(c, pos), &at)) return at;
-        }
-    }
-    while (pos < R) {
+    for (uint32_t pos = 0; pos < R;) {
         uint32_t x[WK], c[WK], mine_n = 0;
 #pragma unroll
         for (uint32_t i = 0; i < WK; ++i) {
@@ -95,13 +68,10 @@ __device__ __forceinline__ uint32_t run_walk(RL_LDS const uint32_t *term, RL_LDS
             mine_n += c[i];
         }
         uint32_t l = 0;       // the lane to go through
-        double nn = 0.0;      // the steps at its start
-        SumSegF g{0, 0.0, 0.0};
-        double scale = 0.0;
         const uint32_t upto_n = wave_incl_u32(mine_n);
         if (s > 0.0) {
-            g = segf_of<P>(s);
-            scale = mul_pow2(1.0, -g.uexp);
+            const SumSegF g = segf_of<P>(s);
+            const double scale = mul_pow2(1.0, -g.uexp);
             StepRun r = run_identity();
 #pragma unroll
             for (uint32_t i = 0; i < WK; ++i)
@@ -123,36 +93,66 @@ __device__ __forceinline__ uint32_t run_walk(RL_LDS const uint32_t *term, RL_LDS
                 continue;
             }
             l = (uint32_t)__builtin_ctzll(evm);
-            nn = g.n + read_lane_f64(ahead, l);
+            s = mul_pow2(g.n + read_lane_f64(ahead, l), g.uexp);
         }
         before += read_lane_u32(upto_n - mine_n, l);
         pos += l * WK;
-        bool crossed = false;
 #pragma unroll
         for (uint32_t i = 0; i < WK; ++i) {
-            if (crossed || pos >= R) continue;
-            const uint32_t xb = read_lane_u32(x[i], l), cnt = read_lane_u32(c[i], l);
-            if (s > 0.0) {
-                // The run's steps from nn, while they stay in the segment.
-                StepRun r = run_identity();
-                run_add_equal(r, xb, cnt, scale);
-                const double e = nn + (r.base + (r.tie ? (double)((parity_of(nn) ^ r.c) & 1u) : 0.0));
-                if (e < g.lim && !pred(mul_pow2(e, g.uexp))) {
-                    nn = e;
-                    before += cnt;
-                    ++pos;
-                    s = mul_pow2(nn, g.uexp);
-                    continue;
-                }
-                s = mul_pow2(nn, g.uexp);
-            }
-            uint32_t at;
-            if (cross(xb, cnt, &at)) return at;
+            if (pos >= R) continue;
+            const uint32_t cnt = read_lane_u32(c[i], l);
+            const uint32_t j = equal_run_walk<P>(s, read_lane_u32(x[i], l), cnt, pred);
+            if (j < cnt) return before + j;
+            before += cnt;
             ++pos;
-            crossed = true;
         }
     }
     return 0xFFFFFFFFu;
+}
+
+// Returns the run whose terms' partial sum first exceeds u, *off the term in it;
+// or R. Written for few instructions, since the code runs once a launch and is
+// fetched cold: with the first runs and four runs a lane written out, the draw
+// took 21 us in f64 and no less in these 32-bit operations; with one run a lane
+// and loops left rolled, here and above, the 256-row call went from 100 to 93 us.
+__device__ __forceinline__ uint32_t run_draw(RL_LDS const uint32_t *term, RL_LDS const uint32_t *n, uint32_t R, float u,
+                                             uint32_t *off) {
+    const uint32_t lane = lane_id();
+    const auto pred = [u](float x) { return x > u; };
+    float s = 0.0f;
+    for (uint32_t pos = 0; pos < R;) {
+        const uint32_t rr = min(pos + lane, R - 1);
+        const uint32_t x = term[rr], c = pos + lane < R ? n[rr] : 0u;
+        uint32_t l = 0;  // the lane whose run holds an event
+        if (s > 0.0f) {
+            const Seg32 g = seg32_of(s);
+            Run32 r{0, 0, 0, 0};
+            if (c != 0) run32_add_equal(r, __uint_as_float(x), c, g.scale);
+            const uint64_t T = ballot(r.tie != 0);
+            uint32_t mine = min(r.base, STEP32_CAP);
+            if (T != 0) {
+                const uint64_t O = ballot(run32_par(r) != 0);
+                uint32_t dep;
+                const uint32_t k = parity_in(T, O, lane, &dep);
+                mine += r.tie ? ((dep ? g.n ^ k : k) ^ r.c) & 1u : 0u;
+            }
+            const uint32_t upto = wave_incl_u32(mine);  // at most 64 (STEP32_CAP + 1): no wrap-around
+            const uint64_t ev = ballot(upto >= (1u << 24) - g.n || pred((float)(g.n + upto) * g.step));
+            l = ev ? (uint32_t)__builtin_ctzll(ev) : WAVE;
+            const uint32_t at = read_lane_u32(upto, min(l, WAVE - 1)) - (ev ? read_lane_u32(mine, l) : 0u);
+            s = (float)(g.n + at) * g.step;
+        }
+        pos += l;
+        if (l == WAVE || pos >= R) continue;
+        const uint32_t cnt = read_lane_u32(c, l);
+        const uint32_t j = equal_run_walk32(s, __uint_as_float(read_lane_u32(x, l)), cnt, pred);
+        if (j < cnt) {
+            *off = j;
+            return pos;
+        }
+        ++pos;
+    }
+    return R;
 }
 
 // Finishes a row from its values' counts (st.values: their window). One
@@ -224,18 +224,13 @@ __device__ __forceinline__ bool finish_values(const RowIO &a, const FullScratch 
     if (nan) L->st_bad = 1;
     __syncthreads();
     if (L->st_bad) return false;
-    if (E <= WAVE) {
-        if (wave == 0) {
-            const uint64_t x = wave_sort64<true>(lane < E ? L->exc[lane] : 0ull);
-            if (lane < E) L->exc[lane] = x;
-        }
-    } else {
-        uint32_t n2 = 1;
-        while (n2 < E) n2 <<= 1;
-        for (uint32_t i = E + tid; i < n2; i += SEL_THREADS) L->exc[i] = 0;
-        __syncthreads();
-        lds_bitonic_desc((RL_LDS uint64_t *)L->exc, n2, SEL_THREADS);
-    }
+    // Each takes the place that the number of elements above it gives.
+    const uint64_t own = tid < E ? L->exc[tid] : 0ull;
+    uint32_t place = 0;
+#pragma unroll 4
+    for (uint32_t i = 0; i < E; ++i) place += L->exc[i] > own ? 1u : 0u;
+    __syncthreads();
+    if (tid < E) L->exc[place] = own;
 
     // ---- the runs in the reference's order ----
     const auto place_key = [lo](uint32_t o) { return total_key(__uint_as_float(val_bits(val_order(o), lo))); };
@@ -274,7 +269,7 @@ __device__ __forceinline__ bool finish_values(const RowIO &a, const FullScratch 
         const uint32_t key = comp_key(L->exc[tid]);
         uint32_t b = 0;  // places whose values are above it
         for (uint32_t h = VAL_BINS / 2; h > 0; h >>= 1)
-                if (place_key(b + h - 1) > key) b += h;
+            if (place_key(b + h - 1) > key) b += h;
         // b <= VAL_BINS - 1: at the last place, -inf, nothing but a NaN below it is missed.
         mine_exc = L->term[b] + tid;
         L->n[mine_exc] = 1;
@@ -283,33 +278,24 @@ __device__ __forceinline__ bool finish_values(const RowIO &a, const FullScratch 
     __syncthreads();
 
     // ---- p, and what the sums' exactness and min-p depend on ----
-    // Thread t holds the runs t per ..
+    // Thread t's runs are r0 .. r1 - 1, in loops that are not unrolled (run_draw).
     const LdsExpTable etab{(RL_LDS uint64_t *)L->exp_tab};
     const TempScale tscale(s.temperature);
     const uint32_t per = (R + SEL_THREADS - 1) / SEL_THREADS;
-    float p[VAL_PER];
-    uint32_t n[VAL_PER];
+    const uint32_t r0 = min(tid * per, R), r1 = min(r0 + per, R);
     double mass_t = 0.0;
     uint32_t n_t = 0;
     PStats ps;
-#pragma unroll
-    for (uint32_t i = 0; i < VAL_PER; ++i) {
-        const uint32_t r = tid * per + i;
-        p[i] = 0.0f;
-        n[i] = 0;
-        if (i < per && r < R) {
-            p[i] = expf_libm_t(tscale(key_value(L->key[r]) - M), etab);
-            n[i] = L->n[r];
-            ps.add(p[i], r, s.min_p);
-            if (p[i] >= s.min_p) ps.count += n[i] - 1;
-            mass_t += (double)p[i] * (double)n[i];
-            n_t += n[i];
-        }
+#pragma unroll 1
+    for (uint32_t r = r0; r < r1; ++r) {
+        const float p = expf_libm_t(tscale(key_value(L->key[r]) - M), etab);
+        const uint32_t n = L->n[r];
+        L->term[r] = __float_as_uint(p);
+        ps.add(p, r, s.min_p);
+        if (p >= s.min_p) ps.count += n - 1;
+        mass_t += (double)p * (double)n;
+        n_t += n;
     }
-    __syncthreads();  // term's first use is over
-#pragma unroll
-    for (uint32_t i = 0; i < VAL_PER; ++i)
-        if (i < per && tid * per + i < R) L->term[tid * per + i] = __float_as_uint(p[i]);
     ps.merge(L);
     double mass;
     const double mass_before = block_exclusive<SEL_THREADS, double>(mass_t, (RL_LDS double *)L->red_d, &mass);
@@ -322,7 +308,7 @@ __device__ __forceinline__ bool finish_values(const RowIO &a, const FullScratch 
     const bool exact = emin > 1000 || mass < mul_pow2(1.0 - 0x1p-30, 30 + emin);
     RL_LDS const uint32_t *term = (RL_LDS const uint32_t *)L->term;
     RL_LDS const uint32_t *occ = (RL_LDS const uint32_t *)L->n;
-    constexpr uint32_t WK = 4;
+    constexpr uint32_t WK = 2;
     const auto never = [](double) { return false; };
 
     // ---- the top-p cut (sample.rs:307-324) ----
@@ -332,28 +318,29 @@ __device__ __forceinline__ bool finish_values(const RowIO &a, const FullScratch 
         const double target = (double)s.top_p * mass;
         double b = mass_before;
         uint32_t nb = n_before, hit = 0xFFFFFFFFu;
-#pragma unroll
-        for (uint32_t i = 0; i < VAL_PER; ++i) {
-            if (hit == 0xFFFFFFFFu && n[i] != 0) {
-                const double x = (double)p[i];
-                if (b + x * (double)n[i] >= target) {
-                    hit = tid * per + i;
+        // Only the thread in whose runs the sum reaches it goes through them.
+        if (b + mass_t >= target && (b < target || tid == 0))
+#pragma unroll 1
+            for (uint32_t r = r0; r < r1; ++r) {
+                const double x = (double)__uint_as_float(L->term[r]);
+                const uint32_t n = L->n[r];
+                if (b + x * (double)n >= target) {
+                    hit = r;
                     // The first of the run's terms to reach it.
                     uint32_t k = 1;
                     if (x > 0.0) {
                         const double d = (target - b) / x;
-                        k = d >= (double)n[i] ? n[i] : d > 1.0 ? (uint32_t)d : 1u;
+                        k = d >= (double)n ? n : d > 1.0 ? (uint32_t)d : 1u;
                     }
                     while (k > 1 && b + x * (double)(k - 1) >= target) --k;
-                    while (k < n[i] && b + x * (double)k < target) ++k;
+                    while (k < n && b + x * (double)k < target) ++k;
                     nb += k;
                     b += x * (double)k;
-                } else {
-                    b += x * (double)n[i];
-                    nb += n[i];
+                    break;
                 }
+                b += x * (double)n;
+                nb += n;
             }
-        }
         if (hit != 0xFFFFFFFFu) atomicMin((uint32_t *)&L->sh_hit, hit);
         __syncthreads();
         if (hit != 0xFFFFFFFFu && L->sh_hit == hit) {
@@ -366,12 +353,12 @@ __device__ __forceinline__ bool finish_values(const RowIO &a, const FullScratch 
     } else {
         if (wave == 0) {
             double sum = 0.0, at_cut = 0.0;
-            run_walk<53, WK>(term, occ, R, never, sum);
+            run_walk<WK>(term, occ, R, never, sum);
             const double target = (double)s.top_p * sum;
             // A target <= 0 is met by the first term.
             uint32_t j = 0;
             if (0.0 >= target) at_cut = (double)__uint_as_float(term[0]);
-            else j = run_walk<53, WK>(term, occ, R, [target](double x) { return x >= target; }, at_cut);
+            else j = run_walk<WK>(term, occ, R, [target](double x) { return x >= target; }, at_cut);
             if (lane == 0) {
                 L->sh_m = j == 0xFFFFFFFFu ? V : j + 1;
                 L->sh_at = at_cut;
@@ -389,15 +376,13 @@ __device__ __forceinline__ bool finish_values(const RowIO &a, const FullScratch 
     // The runs past the m-th candidate end there, for the walks below.
     uint32_t nb = n_before;
     double part = 0.0;
-#pragma unroll
-    for (uint32_t i = 0; i < VAL_PER; ++i) {
-        if (n[i] != 0) {
-            const uint32_t k = nb < m ? min(n[i], m - nb) : 0u;
-            if (k != n[i]) L->n[tid * per + i] = k;
-            part += (double)p[i] * (double)k;
-            if (k != 0 && nb + n[i] >= m) L->sh_run = tid * per + i + 1;  // the runs kept
-            nb += n[i];
-        }
+#pragma unroll 1
+    for (uint32_t r = r0; r < r1; ++r) {
+        const uint32_t n = L->n[r], k = nb < m ? min(n, m - nb) : 0u;
+        if (k != n) L->n[r] = k;
+        part += (double)__uint_as_float(L->term[r]) * (double)k;
+        if (k != 0 && nb + n >= m) L->sh_run = r + 1;  // the runs kept
+        nb += n;
     }
     if (recount && exact) block_exclusive<SEL_THREADS, double>(part, (RL_LDS double *)L->red_d, &total);
     __syncthreads();
@@ -405,7 +390,7 @@ __device__ __forceinline__ bool finish_values(const RowIO &a, const FullScratch 
     if (recount && !exact) {
         if (wave == 0) {
             double sum = 0.0;
-            run_walk<53, WK>(term, occ, Rm, never, sum);
+            run_walk<WK>(term, occ, Rm, never, sum);
             if (lane == 0) L->sh_at = sum;
         }
         __syncthreads();
@@ -413,29 +398,22 @@ __device__ __forceinline__ bool finish_values(const RowIO &a, const FullScratch 
     }
     const float inv = (float)(1.0 / total);
     if (!(inv <= 3.40282347e38f)) return false;
-#pragma unroll
-    for (uint32_t i = 0; i < VAL_PER; ++i)
-        if (n[i] != 0) L->term[tid * per + i] = __float_as_uint(p[i] * inv);
+    for (uint32_t r = tid; r < Rm; r += SEL_THREADS) L->term[r] = __float_as_uint(__uint_as_float(L->term[r]) * inv);
     __syncthreads();
 
     // ---- the draw (sample.rs:349-358) ----
     if (wave == 0) {
         const float u = a.uniforms[row];
-        double sum = 0.0;
-        const uint32_t j = 0.0 > (double)u ? 0u
-                                           : run_walk<24, WK>(term, occ, Rm, [u](double x) { return x > (double)u; }, sum);
-        if (lane == 0) L->sh_pick = j < m ? j : m - 1;
-    }
-    __syncthreads();
-    const uint32_t pick = L->sh_pick;
-    nb = n_before;
-#pragma unroll
-    for (uint32_t i = 0; i < VAL_PER; ++i) {
-        if (n[i] != 0 && pick - nb < n[i]) {
-            L->sh_run = tid * per + i;
-            L->sh_off = pick - nb;
+        uint32_t off = 0;
+        uint32_t r = 0.0f > u ? 0u : run_draw(term, occ, Rm, u, &off);
+        if (r == Rm) {  // a shortfall takes the last candidate
+            r = Rm - 1;
+            off = occ[r] - 1;
         }
-        nb += n[i];
+        if (lane == 0) {
+            L->sh_run = r;
+            L->sh_off = off;
+        }
     }
     __syncthreads();
     const uint32_t run = L->sh_run, off = L->sh_off;

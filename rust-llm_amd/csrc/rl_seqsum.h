@@ -399,6 +399,115 @@ RL_HD inline uint32_t equal_run_walk(double &s, uint32_t xb, uint32_t count, Pre
     return count;
 }
 
+// ---- f32 sums in 32-bit arithmetic ----
+// The same grid, steps and runs for P = 24 and a normal sum above 2^-60, whose
+// counts fit 32 bits: a draw's sums of a few thousand runs are one chain of
+// these operations, and f64 ones are several times longer.
+constexpr uint32_t STEP32_CAP = 1u << 25;  // a run's steps, cut: above any segment's room (2^24)
+
+struct Seg32 {
+    uint32_t n;         // the sum is n steps, 2^23 <= n < 2^24
+    float step, scale;  // a step, and steps per unit (powers of two)
+};
+
+// s: a normal f32 in [2^-60, 2^60].
+RL_HD inline Seg32 seg32_of(float s) {
+    uint32_t b;
+    memcpy(&b, &s, 4);
+    Seg32 g;
+    const uint32_t e = b >> 23;  // biased
+    g.n = (b & 0x7FFFFFu) | 0x800000u;
+    g.step = f32_from_bits((e - 23u) << 23);
+    g.scale = f32_from_bits((277u - e) << 23);  // 2^(23 - (e - 127))
+    return g;
+}
+
+// A term's steps when it is not an exact tie (then rounded down), at most STEP32_CAP.
+RL_HD inline uint32_t step32_of(float x, float scale, bool *tie) {
+    float y = x * scale;
+    y = y < (float)STEP32_CAP ? y : (float)STEP32_CAP;
+    const float fl = __builtin_floorf(y), fr = y - fl;
+    *tie = fr == 0.5f;
+    return (uint32_t)fl + (fr > 0.5f ? 1u : 0u);
+}
+
+RL_HD inline uint32_t mul32_cut(uint32_t a, uint32_t b) {
+    const uint64_t c = (uint64_t)a * b;
+    return c < STEP32_CAP ? (uint32_t)c : STEP32_CAP;
+}
+
+// StepRun with counts cut at STEP32_CAP by the caller; a run that is cut is
+// only known to leave the segment.
+struct Run32 {
+    uint32_t base, mark, tie, c;
+};
+
+// Appends n >= 1 equal terms, as run_add_equal.
+RL_HD inline void run32_add_equal(Run32 &r, float x, uint32_t n, float scale) {
+    bool t;
+    const uint32_t q = step32_of(x, scale, &t);
+    if (!t) {
+        r.base += mul32_cut(q, n);
+        return;
+    }
+    const uint32_t pq = q & 1u;
+    if (!r.tie) {
+        r.tie = 1;
+        r.c = (r.base ^ pq) & 1u;
+        r.base += q;
+    } else {
+        r.base += q + (((r.base - r.mark) ^ pq) & 1u);
+    }
+    r.base += mul32_cut(q + pq, n - 1);
+    r.mark = r.base;
+}
+RL_HD inline uint32_t run32_par(const Run32 &r) { return (r.tie ? r.base - r.mark : r.base) & 1u; }
+
+// equal_run_walk for P = 24, a sum that is 0 or in [2^-60, 2^60], and a term
+// below 2^60 (from 0 the first term x >= 2^-60).
+template <class Pred>
+RL_HD inline uint32_t equal_run_walk32(float &s, float x, uint32_t count, Pred pred) {
+    uint32_t done = 0;
+    while (done < count) {
+        if (s > 0.0f) {
+            const Seg32 g = seg32_of(s);
+            bool tie;
+            const uint32_t q = step32_of(x, g.scale, &tie), pq = q & 1u;
+            const uint32_t first = tie ? q + ((g.n ^ pq) & 1u) : q, rest = tie ? q + pq : q;
+            const uint32_t room = (1u << 24) - g.n, left = count - done;
+            if (first < room) {
+                // K: the terms whose sums stay below the segment's end.
+                const uint32_t a = room - first;
+                uint32_t K = left;
+                if (rest != 0) {
+                    const uint32_t most = (a + rest - 1) / rest;
+                    K = most < left ? most : left;
+                }
+                auto sum_at = [&](uint32_t j) { return (float)(g.n + first + (j - 1) * rest) * g.step; };
+                if (pred(sum_at(K))) {
+                    uint32_t lo = 1, hi = K;
+                    while (lo < hi) {
+                        const uint32_t mid = lo + (hi - lo) / 2;
+                        if (pred(sum_at(mid)))
+                            hi = mid;
+                        else
+                            lo = mid + 1;
+                    }
+                    s = sum_at(lo);
+                    return done + (lo - 1);
+                }
+                s = sum_at(K);
+                done += K;
+                if (done == count) return count;
+            }
+        }
+        s = s + x;  // this term's sum leaves the segment
+        if (pred(s)) return done;
+        ++done;
+    }
+    return count;
+}
+
 #if defined(__HIPCC__)
 // ------------------------------------------------------------- device ---
 // LDS a workgroup of NT threads needs for seq_replay. The per-wave records

@@ -505,8 +505,59 @@ static void check_add_equal(int &cases) {
     }
 }
 
+// The 32-bit forms against the plain f32 loop: equal_run_walk32's sums and
+// first indices, and run32_add_equal's counts and parities against StepRun's
+// below the cut.
+static void check_runs32(int &cases) {
+    for (int rep = 0; rep < 6000; ++rep) {
+        const float s0 = rep % 5 == 0 ? 0.0f : (float)ldexp(unit() + 0.5, -(int)(rnd() % 22));
+        const int gx = s0 > 0.0f ? seg_of<24>(s0).uexp : -45;
+        float x;
+        switch (rnd() % 5) {
+        case 0: x = (float)ldexp((double)(2 * (rnd() % 64) + 1), gx - 1); break;
+        case 1: x = (float)ldexp((double)(rnd() % 4096), gx); break;
+        case 2: x = (float)ldexp(unit(), gx - 3); break;
+        case 3: x = (float)(s0 * (1.0 + 4.0 * unit())); break;
+        default: x = (float)ldexp(unit() + 0.5, -(int)(rnd() % 30) - 4); break;
+        }
+        if (s0 == 0.0f && !(x >= 0x1p-50f)) x = 0x1p-21f;
+        const uint32_t n = 1 + (uint32_t)(rnd() % (rep % 10 == 0 ? 300000 : 300));
+        std::vector<float> partial(n);
+        float a = s0;
+        for (uint32_t i = 0; i < n; ++i) partial[i] = a = a + x;
+        for (int k = 0; k < 4; ++k) {
+            const float thr = k == 0 ? 2.0f * a + 1.0f : k == 1 ? -1.0f : partial[rnd() % n];
+            float s = s0;
+            const uint32_t got = equal_run_walk32(s, x, n, [thr](float v) { return v > thr; });
+            uint32_t want = 0;
+            while (want < n && !(partial[want] > thr)) ++want;
+            if (got != want || s != partial[want < n ? want : n - 1]) {
+                ++failures;
+                printf("FAIL runs32: rep %d n %u got %u want %u\n", rep, n, got, want);
+            }
+            ++cases;
+        }
+        if (s0 > 0.0f) {
+            const Seg32 g = seg32_of(s0);
+            Run32 r{0, 0, 0, 0};
+            StepRun d = run_identity();
+            for (int k = 0; k < 3; ++k) {
+                const float y = (float)ldexp((double)(rnd() % 512), gx - 1);
+                const uint32_t m = 1 + (uint32_t)(rnd() % 2000);
+                run32_add_equal(r, y, m, g.scale);
+                run_add_equal(d, fbits(y), m, ldexp(1.0, -gx));
+            }
+            if ((double)r.base != d.base || r.tie != d.tie || run32_par(r) != run_par(d) || (r.tie && r.c != d.c)) {
+                ++failures;
+                printf("FAIL runs32 counts: rep %d\n", rep);
+            }
+        }
+    }
+}
+
 int main() {
     int cases = 0;
+    check_runs32(cases);
     check_assoc();
     check_runs();
     check_add_equal(cases);
