@@ -36,7 +36,8 @@ constexpr uint32_t MAX_VOCAB = 1u << 21;
 constexpr uint32_t TARGET_WGS = 1024;  // enough workgroups to cover 256 CUs four deep
 constexpr uint32_t FULL_GROUP_MAX = 256;
 constexpr uint32_t CHUNK_SLOTS = 2 * TARGET_WGS;
-constexpr uint32_t SEL_TARGET_WGS = 512;
+constexpr uint32_t SEL_PASS_WGS = 512;
+constexpr uint32_t SEL_TARGET_WGS = 256;
 constexpr uint32_t SEL_HEAD_WGS = 256;
 static_assert((MAX_VOCAB + SEL_CHUNK_MAX - 1) / SEL_CHUNK_MAX <= MAX_CHUNKS, "the gather's chunks");
 
@@ -573,13 +574,19 @@ int rl_sampler_sample_rows(rl_sampler_ctx *ctx, const float *logits, uint64_t ro
         f.row0 = ctx->full_rows[g0];
         // Rows of the group that take the selection path: with any, the pass
         // counts bins and the gather runs; with no others, few rows are read
-        // in more chunks.
+        // in more chunks. With no others the pass takes half the workgroups:
+        // each ends with its bins' device-scope adds (24 x 151935 at top-p
+        // 0.9 52 -> 48 us a call, 40 x 248320 at top-k 100 60 -> 54 with the
+        // gather's below, one to four rows the same).
         const uint32_t nsel = ctx->select_upto[g0 + ng - 1] - (g0 ? ctx->select_upto[g0 - 1] : 0u);
         const uint32_t most = nsel == ng ? FULL_CHUNKS : MAX_CHUNKS;
-        f.chunks = std::max(1u, std::min(most, (TARGET_WGS + ng - 1) / ng));
+        const uint32_t pass_wgs = nsel == ng ? SEL_PASS_WGS : TARGET_WGS;
+        f.chunks = std::max(1u, std::min(most, (pass_wgs + ng - 1) / ng));
         f.chunks = std::min(f.chunks, std::max(1u, vocab / 4096));
-        // The gather's chunks: two workgroups a CU while rows are few, each of
-        // at least a float4 a thread, at most SEL_CHUNK_MAX elements.
+        // The gather's chunks: a workgroup a CU while rows are few, each of at
+        // least a float4 a thread, at most SEL_CHUNK_MAX elements. Two a CU
+        // start late (sixteen waves each): 16 x 248320 at top-k 100 47 us a
+        // call with 512, 42 with 256, 43 with 192.
         uint32_t gchunks = std::max(1u, std::min({FULL_CHUNKS, SEL_TARGET_WGS / ng, vocab / (4 * SEL_THREADS)}));
         gchunks = std::max(gchunks, (vocab + SEL_CHUNK_MAX - 1) / SEL_CHUNK_MAX);
         FullScratch fs{ctx->d_keyA,     ctx->d_idA,      ctx->d_keyB,     ctx->d_idB,        ctx->d_probs,
