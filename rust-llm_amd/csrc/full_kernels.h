@@ -18,8 +18,6 @@
 // sequential rounding in parallel. Rows with a NaN or infinite p (NaN logits,
 // a NaN temperature, 1 / total overflowing) are walked in order by one thread.
 #pragma once
-#include <type_traits>
-
 #include "minp_bound.h"
 #include "sampler_kernels.h"
 #include "select_bins.h"
@@ -331,53 +329,16 @@ __device__ __forceinline__ bool finish_wave(const RowIO &a, uint32_t row, const 
     return true;
 }
 
-constexpr uint32_t DRAW_BLOCK = 32;
-
-// The draw (sample.rs:349-358) over the m terms q[0..m) in LDS: the index of
-// the first whose running f32 sum exceeds u, or m - 1. q is 16-byte aligned and
-// holds zeros from m to the next multiple of DRAW_BLOCK. One wave, every lane
-// alike: the sum is one chain of additions, so the rest is kept off it: the
-// next block's reads are in flight, and only a block's last sum is compared
-// (the sums never fall).
-__device__ __forceinline__ uint32_t draw_walk(RL_LDS const uint32_t *q, uint32_t m, float u) {
-    typedef float vf4 __attribute__((ext_vector_type(4)));
-    vf4 nx[DRAW_BLOCK / 4];
-#pragma unroll
-    for (uint32_t i = 0; i < DRAW_BLOCK / 4; ++i) nx[i] = *(RL_LDS const vf4 *)&q[4 * i];
-    float run = 0.0f;
-    for (uint32_t j = 0; j < m; j += DRAW_BLOCK) {
-        vf4 x[DRAW_BLOCK / 4];
-#pragma unroll
-        for (uint32_t i = 0; i < DRAW_BLOCK / 4; ++i) x[i] = nx[i];
-        const uint32_t jn = j + DRAW_BLOCK < m ? j + DRAW_BLOCK : j;
-#pragma unroll
-        for (uint32_t i = 0; i < DRAW_BLOCK / 4; ++i) nx[i] = *(RL_LDS const vf4 *)&q[jn + 4 * i];
-        float c = run;
-#pragma unroll
-        for (uint32_t i = 0; i < DRAW_BLOCK; ++i) c += x[i / 4][i & 3u];
-        if (c > u) {
-            c = run;
-            uint32_t hit = DRAW_BLOCK;
-#pragma unroll
-            for (uint32_t i = 0; i < DRAW_BLOCK; ++i) {
-                c += x[i / 4][i & 3u];
-                if (hit == DRAW_BLOCK && c > u) hit = i;
-            }
-            return min(j + hit, m - 1);
-        }
-        run = c;
-    }
-    return m - 1;
-}
-
 // The same finish for 64 < c <= FIN_CAP survivors: sv holds their
 // keep_order composites, sorted here by the workgroup (NT threads); sp gets
-// their p, and room up to the next multiple of DRAW_BLOCK. One wave replays the
-// reference's sums in order (the f64 cut and total, the f32 draw) from LDS
-// reads that run ahead of the additions, and the workgroup writes the kept
+// their p. One wave replays the sums in order (the f64 cut and total, the f32
+// draw), 64 terms in its lanes at a time, and the workgroup writes the kept
 // candidates. Every thread returns the same verdict. A row of 75 survivors
 // among 64 rows of a few makes the call as slow as its finish: one thread
-// walking the list after a sorting network took 18 us, half of the call.
+// walking the list after a sorting network took 18 us, half of the call. The
+// walks are short loops: written out for reads ahead of the additions they were
+// no faster at 75, and their code cost a call of one row, which never runs it,
+// 0.5 us.
 template <uint32_t NT>
 __device__ __forceinline__ bool finish_block(const RowIO &a, uint32_t row, const rl_sampling &s, float M, uint32_t c,
                                              RL_LDS uint64_t *sv, RL_LDS float *sp, RL_LDS uint32_t *sh,
@@ -406,25 +367,28 @@ __device__ __forceinline__ bool finish_block(const RowIO &a, uint32_t row, const
     __syncthreads();
     if (wave == 0) {
         // sh[0]: kept (0 when the row is left to k_full_rest), sh[1]: a q that is not finite.
-        RL_LDS const uint32_t *pw = (RL_LDS const uint32_t *)sp;
-        uint32_t kept = c;
+        // The first sum to reach `stop`: t_lo for the top-p cut, which is
+        // certain when that sum reaches t_hi too; the first sum of all for a
+        // top_p <= 0 (sample.rs:315-323); none in id order.
+        const bool cut = !by_id && s.top_p > 0.0f;
+        const double stop = cut ? t_lo : by_id ? __builtin_inf() : -__builtin_inf();
         double total = 0.0;
-        bool ok = true;
-        if (by_id) {
-            seq_walk<53>(pw, c, NeverStop(), total);
-        } else if (ns_key != 0 && !(keep_key(sv[c - 1], false) >= ns_key)) {
-            ok = false;
-        } else if (!(s.top_p > 0.0f)) {
-            kept = 1;  // sample.rs:315-323
-            total = (double)sp[0];
-        } else {
-            // The first sum to reach t_lo; the cut is certain when it reaches t_hi too.
-            const uint32_t j = seq_walk<53>(pw, c, [t_lo](double x) { return x >= t_lo; }, total);
-            if (j < c) {
-                ok = total >= t_hi;
-                kept = j + 1;
+        uint32_t kept = c;
+        for (uint32_t b0 = 0; b0 < c && kept == c; b0 += WAVE) {
+            const float p = sp[min(b0 + tid, c - 1)];
+            const uint32_t nb = min(WAVE, c - b0);
+#pragma unroll 1
+            for (uint32_t i = 0; i < nb; ++i) {
+                total += (double)read_lane_f32(p, i);
+                if (total >= stop) {
+                    kept = b0 + i + 1;
+                    break;
+                }
             }
+            if (total >= stop) break;
         }
+        bool ok = !(cut && total >= t_lo && !(total >= t_hi));
+        if (!by_id && ns_key != 0 && !(keep_key(sv[c - 1], false) >= ns_key)) ok = false;
         if (tid == 0) {
             sh[0] = ok ? kept : 0u;
             *sh_inv = (float)(1.0 / total);
@@ -434,9 +398,8 @@ __device__ __forceinline__ bool finish_block(const RowIO &a, uint32_t row, const
     const uint32_t kept = sh[0];
     if (kept == 0) return false;
     const float inv = *sh_inv;
-    const uint32_t padded = (kept + DRAW_BLOCK - 1) / DRAW_BLOCK * DRAW_BLOCK;
-    for (uint32_t i = tid; i < padded; i += NT) {
-        const float q = i < kept ? sp[i] * inv : 0.0f;
+    for (uint32_t i = tid; i < kept; i += NT) {
+        const float q = sp[i] * inv;
         if (!(q <= 3.40282347e38f)) sh[1] = 1;
         sp[i] = q;
     }
@@ -444,7 +407,20 @@ __device__ __forceinline__ bool finish_block(const RowIO &a, uint32_t row, const
     if (sh[1]) return false;
     if (wave == 0) {
         // The draw, while the other waves write the candidates.
-        const uint32_t pick = draw_walk((RL_LDS const uint32_t *)sp, kept, u);
+        float cum = 0.0f;
+        uint32_t pick = kept - 1;
+        for (uint32_t b0 = 0; b0 < kept && !(cum > u); b0 += WAVE) {
+            const float q = sp[min(b0 + tid, kept - 1)];
+            const uint32_t nb = min(WAVE, kept - b0);
+#pragma unroll 1
+            for (uint32_t i = 0; i < nb; ++i) {
+                cum += read_lane_f32(q, i);
+                if (cum > u) {
+                    pick = b0 + i;
+                    break;
+                }
+            }
+        }
         if (tid == 0) {
             a.out_token[row] = keep_id(sv[pick], by_id);
             a.out_kept[row] = kept;
@@ -649,21 +625,20 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
     double S = 0.0;                   // per lane: mass relative to m_run
     uint32_t first_inf = 0xFFFFFFFFu;
     bool nan_seen = false;
-    // The penalised logit of element e of this chunk, from memory (rare paths).
+    // The penalised logit of element e of this chunk, re-read from memory
+    // (the candidates' rare path; their row was just read).
     auto value_at = [&](uint32_t e) {
         float v = ((const RL_GLB float *)rowp)[e];
         if (pen && ((bm[(e - e0) >> 5] >> ((e - e0) & 31)) & 1u)) v = penalize(v, s.repeat_penalty);
         return v;
     };
-    // Appends this lane's candidates (the set bits i < N of mb, of values
-    // val_of(i) and vocabulary ids id_of(i)) to the chunk's LDS buffer: one LDS
-    // atomic per wave, slots by an exclusive scan of the lanes' counts. The
-    // values come from the step's registers, one test an element: read again
-    // from memory, a load after another while a lane held several, they cost
-    // most of the 64-row zipf pass's time. A full buffer sends the row to
-    // k_full_rest.
-    auto append = [&](uint64_t mb, auto n_of, auto val_of, auto id_of) {
-        constexpr uint32_t N = decltype(n_of)::value;
+    // Appends this lane's candidates (the set bits i of mb; id_of(i) is the
+    // vocabulary id of candidate i) to the chunk's LDS buffer: one LDS atomic
+    // per wave, slots by an exclusive scan of the lanes' counts. The values are
+    // read again (from the caches): taken from the step's registers, a test an
+    // element, they cost a call of few rows 1 us more than that, since the code
+    // runs once and is fetched cold. A full buffer sends the row to k_full_rest.
+    auto append = [&](uint64_t mb, auto id_of) {
         const uint32_t mine = (uint32_t)__popcll(mb);
         const uint32_t incl = wave_incl_u32(mine);
         const uint32_t wtotal = (uint32_t)__builtin_amdgcn_readlane((int)incl, WAVE - 1);
@@ -672,18 +647,19 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
         base = (uint32_t)__builtin_amdgcn_readlane((int)base, 0);
         if (base + wtotal > PASS_CAND) {
             // The buffer is full: the row leaves the min-p path, and nothing
-            // more is listed for it.
+            // more is listed (or re-read) for it.
             if (lane == 0) sh_cover = 1;
             mass = false;
             return;
         }
         uint32_t at = base + incl - mine;
-#pragma unroll
-        for (uint32_t i = 0; i < N; ++i)
-            if ((mb >> i) & 1ull) cbuf[at++] = composite(total_key(val_of(i)), id_of(i));
+        while (mb != 0) {
+            const uint32_t i = (uint32_t)__ffsll((unsigned long long)mb) - 1u;
+            mb &= mb - 1ull;
+            const uint32_t e = id_of(i);
+            cbuf[at++] = composite(total_key(value_at(e)), e);
+        }
     };
-    const auto of_step = std::integral_constant<uint32_t, 4 * PASS_U>();
-    const auto of_one = std::integral_constant<uint32_t, 1>();
     // Counts element x into its bin (select rows).
     auto count = [&](float x) {
         float edge;
@@ -730,8 +706,7 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
                     }
                 }
                 if (ballot(mb != 0) != 0 && sh_cover == 0)
-                    append(mb, of_step, [&](uint32_t i) { return A[i >> 2][i & 3u]; },
-                           [&](uint32_t i) { return 4 * (b + (i >> 2) * FULL_THREADS + tid) + (i & 3u); });
+                    append(mb, [&](uint32_t i) { return 4 * (b + (i >> 2) * FULL_THREADS + tid) + (i & 3u); });
             }
             if (chunk == C - 1) {  // the last vocab % 4 elements
                 const uint32_t e = 4 * n4 + tid;
@@ -740,7 +715,7 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
                 if (ok) tmax = fmaxf(tmax, x);
                 const uint64_t mb = ok && !count_value(x) ? 1ull : 0ull;
                 if (ballot(mb != 0) != 0 && sh_cover == 0)
-                    append(mb, of_one, [&](uint32_t) { return x; }, [&](uint32_t) { return e; });
+                    append(mb, [&](uint32_t) { return e; });
             }
             m_run = uniform_f32(wave_maxnum_f32(tmax));
             if (m_run == __builtin_inff())  // this wave's first +inf (among others'; the row takes the lowest)
@@ -838,8 +813,7 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
                     for (uint32_t c = 0; c < 4; ++c)
                         if (ok && (A[u][c] - m_run) * c2 >= zthr) mb |= 1ull << (4 * u + c);
                 }
-                append(mb, of_step, [&](uint32_t i) { return A[i >> 2][i & 3u]; },
-                       [&](uint32_t i) { return 4 * (b + (i >> 2) * FULL_THREADS + tid) + (i & 3u); });
+                append(mb, [&](uint32_t i) { return 4 * (b + (i >> 2) * FULL_THREADS + tid) + (i & 3u); });
             }
         } else if (eligible && m_run == -__builtin_inff()) {
             // Nothing finite so far: no mass, but a NaN must still send the
@@ -874,7 +848,7 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
             const float z = (xe - m_run) * c2;
             if (ok) S += (double)__builtin_amdgcn_exp2f(z);
             const uint64_t mb = (ok && z >= zthr) ? 1ull : 0ull;
-            if (ballot(mb != 0) != 0) append(mb, of_one, [&](uint32_t) { return xe; }, [&](uint32_t) { return e; });
+            if (ballot(mb != 0) != 0) append(mb, [&](uint32_t) { return e; });
         } else if (eligible && ok && xe != xe) {
             nan_seen = true;
         }

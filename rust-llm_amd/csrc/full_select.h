@@ -18,9 +18,9 @@
 //
 // Before, k_full_rest sorted every such row: four radix passes over the
 // vocabulary on one CU. A call over one row of 248 320 at top-p 0.95 went from
-// 1340 to 37 us, 24 unaligned rows of 151 935 at top-p 0.9 from 904 to 56 us,
-// 16 rows of 248 320 at top-k 100 from 933 to 46 us. What bounds it now: four
-// launches and, in each, one chain of dependent steps (about 9, 9, 13 and 2 us
+// 1348 to 37 us, 24 unaligned rows of 151 935 at top-p 0.9 from 897 to 48 us,
+// 16 rows of 248 320 at top-k 100 from 931 to 40 us. What bounds it now: four
+// launches and, in each, one chain of dependent steps (about 11, 9, 10 and 2 us
 // at one row); the logits' two reads are a small part.
 //
 // Measured and not kept: the finish in the gather's last chunk to arrive (the
@@ -331,6 +331,8 @@ __device__ __forceinline__ void count_sort(uint64_t x, uint32_t n, RL_LDS uint64
 }
 
 // --------------------------------------------------------- the finish ---
+constexpr uint32_t DRAW_BLOCK = 32;
+
 struct FinishLds {
     uint64_t v[SEL_FIN_CAP];                  // the elements, sorted
     __attribute__((aligned(16))) uint32_t p[SEL_FIN_CAP + DRAW_BLOCK];  // their p, then q (f32 words)
@@ -342,6 +344,43 @@ struct FinishLds {
     uint32_t sh_hit, sh_in, sh_out;
     double sh_at;
 };
+
+// The draw (sample.rs:349-358) over the m terms q[0..m) in LDS: the index of
+// the first whose running f32 sum exceeds u, or m - 1. q is 16-byte aligned and
+// holds zeros from m to the next multiple of DRAW_BLOCK. One wave, every lane
+// alike: the sum is one chain of additions, so the rest is kept off it: the
+// next block's reads are in flight, and only a block's last sum is compared
+// (the sums never fall).
+__device__ __forceinline__ uint32_t draw_walk(RL_LDS const uint32_t *q, uint32_t m, float u) {
+    typedef float vf4 __attribute__((ext_vector_type(4)));
+    vf4 nx[DRAW_BLOCK / 4];
+#pragma unroll
+    for (uint32_t i = 0; i < DRAW_BLOCK / 4; ++i) nx[i] = *(RL_LDS const vf4 *)&q[4 * i];
+    float run = 0.0f;
+    for (uint32_t j = 0; j < m; j += DRAW_BLOCK) {
+        vf4 x[DRAW_BLOCK / 4];
+#pragma unroll
+        for (uint32_t i = 0; i < DRAW_BLOCK / 4; ++i) x[i] = nx[i];
+        const uint32_t jn = j + DRAW_BLOCK < m ? j + DRAW_BLOCK : j;
+#pragma unroll
+        for (uint32_t i = 0; i < DRAW_BLOCK / 4; ++i) nx[i] = *(RL_LDS const vf4 *)&q[jn + 4 * i];
+        float c = run;
+#pragma unroll
+        for (uint32_t i = 0; i < DRAW_BLOCK; ++i) c += x[i / 4][i & 3u];
+        if (c > u) {
+            c = run;
+            uint32_t hit = DRAW_BLOCK;
+#pragma unroll
+            for (uint32_t i = 0; i < DRAW_BLOCK; ++i) {
+                c += x[i / 4][i & 3u];
+                if (hit == DRAW_BLOCK && c > u) hit = i;
+            }
+            return min(j + hit, m - 1);
+        }
+        run = c;
+    }
+    return m - 1;
+}
 
 // The finish of a row of n <= SEL_FIN_CAP collected elements by one
 // workgroup: L->v holds them sorted, tail is the sum of every other p (0 for
