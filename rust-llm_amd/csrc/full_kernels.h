@@ -375,17 +375,22 @@ __device__ __forceinline__ bool finish_block(const RowIO &a, uint32_t row, const
         double total = 0.0;
         uint32_t kept = c;
         for (uint32_t b0 = 0; b0 < c && kept == c; b0 += WAVE) {
-            const float p = sp[min(b0 + tid, c - 1)];
-            const uint32_t nb = min(WAVE, c - b0);
-#pragma unroll 1
-            for (uint32_t i = 0; i < nb; ++i) {
-                total += (double)read_lane_f32(p, i);
-                if (total >= stop) {
-                    kept = b0 + i + 1;
-                    break;
-                }
+            const float p = b0 + tid < c ? sp[b0 + tid] : 0.0f;
+            // Four terms a test (the sums never fall), then the one that reaches it.
+            uint32_t i = 0;
+            for (; i < WAVE && b0 + i < c; i += 4) {
+                double t = total;
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) t += (double)read_lane_f32(p, i + k);
+                if (t >= stop) break;
+                total = t;
             }
-            if (total >= stop) break;
+            if (i < WAVE && b0 + i < c) {
+                do total += (double)read_lane_f32(p, i++);
+                while (!(total >= stop));
+                kept = b0 + i;
+                break;
+            }
         }
         bool ok = !(cut && total >= t_lo && !(total >= t_hi));
         if (!by_id && ns_key != 0 && !(keep_key(sv[c - 1], false) >= ns_key)) ok = false;
@@ -410,15 +415,19 @@ __device__ __forceinline__ bool finish_block(const RowIO &a, uint32_t row, const
         float cum = 0.0f;
         uint32_t pick = kept - 1;
         for (uint32_t b0 = 0; b0 < kept && !(cum > u); b0 += WAVE) {
-            const float q = sp[min(b0 + tid, kept - 1)];
-            const uint32_t nb = min(WAVE, kept - b0);
-#pragma unroll 1
-            for (uint32_t i = 0; i < nb; ++i) {
-                cum += read_lane_f32(q, i);
-                if (cum > u) {
-                    pick = b0 + i;
-                    break;
-                }
+            const float q = b0 + tid < kept ? sp[b0 + tid] : 0.0f;
+            uint32_t i = 0;
+            for (; i < WAVE && b0 + i < kept; i += 4) {
+                float t = cum;
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) t += read_lane_f32(q, i + k);
+                if (t > u) break;
+                cum = t;
+            }
+            if (i < WAVE && b0 + i < kept) {
+                do cum += read_lane_f32(q, i++);
+                while (!(cum > u));
+                pick = b0 + i - 1;
             }
         }
         if (tid == 0) {
