@@ -79,13 +79,7 @@ __device__ __forceinline__ bool identity_order(const rl_sampling &s, uint32_t V)
     return full_k(s, V) == V && !(s.top_p < 1.0f);  // no select and no sort
 }
 
-// Chunk c of n items split into `chunks`: [chunk_lo(c), chunk_lo(c + 1)).
-// Callers split a row's float4 (n <= 2^19, the vocabulary being at most 2^21)
-// into at most FULL_CHUNKS, so n * c fits 32 bits.
-static_assert((uint64_t)FULL_CHUNKS * (1u << 19) < (1ull << 32), "chunk bounds in 32 bits");
-__device__ __forceinline__ uint32_t chunk_lo(uint32_t n, uint32_t c, uint32_t chunks) {
-    return n * c / chunks;
-}
+static_assert((uint64_t)FULL_CHUNKS * (1u << 19) < (1ull << 32), "chunk_lo in 32 bits");
 
 // The argument (l - max) / t of the reference's p = exp((l - max) / t)
 // (sample.rs:309). When t is a power of two with a normal reciprocal, the
@@ -110,11 +104,9 @@ __device__ __forceinline__ bool small_eligible(const rl_sampling &s, uint32_t V)
     return s.min_p > 0.0f && full_k(s, V) == V && s.temperature > 0.0f;
 }
 
-// Whether a row takes the selection path (full_select.h): it keeps the head of
-// the descending order, by top-k (top_k < vocab), or by top-p alone over the
-// whole vocabulary (with min-p on it tries the min-p path).
-__device__ __forceinline__ bool select_eligible(const rl_sampling &s, uint32_t V) {
-    return s.temperature > 0.0f && (full_k(s, V) < V || (s.top_p < 1.0f && !(s.min_p > 0.0f)));
+// Whether a row takes the selection path.
+__host__ __device__ inline bool select_eligible(const rl_sampling &s, uint32_t V) {
+    return sel_takes(s.temperature, s.top_k, s.top_p, s.min_p, V);
 }
 
 // A value row's counts of each value in a chunk: VAL_BINS / 2 words of two. The

@@ -44,7 +44,6 @@ constexpr uint32_t SEL_WAVES = SEL_THREADS / WAVE;
 constexpr uint32_t SEL_FIN_CAP = SEL_GROUP;          // elements finished in LDS
 constexpr uint32_t SEL_U = 2;                        // float4 per thread per step of the gather
 constexpr uint32_t SEL_STEP = SEL_THREADS * SEL_U;   // float4 per step
-constexpr uint32_t SEL_CHUNK_MAX = 65536;            // most float4-whole elements of a chunk (a window bitmap of 8 KiB)
 constexpr uint32_t SORT_BUCKETS = 4096;
 constexpr uint32_t SORT_CROWD = 192;                 // a bucket above this is sorted by the network
 
@@ -738,6 +737,7 @@ __global__ __launch_bounds__(SEL_THREADS) void k_full_gather(RowIO a, FullScratc
     }
     const uint64_t tab = EXP2_32_TAB[tid & 31u];
     f32x4 nx[SEL_U];
+    // A chunk holds a float4 (sel_gather_chunks): q1 - 1 is one of its own.
     auto fetch = [&](uint32_t b) {
 #pragma unroll
         for (uint32_t u = 0; u < SEL_U; ++u) {

@@ -62,13 +62,6 @@ Path plan_row(const rl_sampling &s, uint32_t vocab) {
     return Path::Full;
 }
 
-// Whether a full-path row may take the selection path (select_eligible of
-// full_kernels.h, which the kernels decide by).
-bool takes_selection(const rl_sampling &s, uint32_t vocab) {
-    const bool by_k = s.top_k != 0 && s.top_k < vocab;
-    return s.temperature > 0.0f && (by_k || (s.top_p < 1.0f && !(s.min_p > 0.0f)));
-}
-
 uint64_t row_cand_need(const rl_sampling &s, uint32_t vocab) {
     if (s.temperature <= 0.0f) return 1;
     if (s.top_k == 0 || s.top_k >= vocab) return vocab;
@@ -395,7 +388,7 @@ int rl_sampler_configure(rl_sampler_ctx *ctx, const rl_sampling *settings, uint3
         (p == Path::Greedy ? ctx->greedy_rows : p == Path::Stream ? ctx->stream_rows : ctx->full_rows).push_back(r);
         if (p == Path::Full) {
             const uint32_t before = ctx->select_upto.empty() ? 0u : ctx->select_upto.back();
-            ctx->select_upto.push_back(before + (takes_selection(settings[r], ctx->vocab) ? 1u : 0u));
+            ctx->select_upto.push_back(before + (select_eligible(settings[r], ctx->vocab) ? 1u : 0u));
         }
         need = std::max(need, row_cand_need(settings[r], ctx->vocab));
         ctx->need_upto.push_back(need);
@@ -591,8 +584,7 @@ int rl_sampler_sample_rows(rl_sampler_ctx *ctx, const float *logits, uint64_t ro
         // least a float4 a thread, at most SEL_CHUNK_MAX elements. Two a CU
         // start late (sixteen waves each): 16 x 248320 at top-k 100 47 us a
         // call with 512, 42 with 256, 43 with 192.
-        uint32_t gchunks = std::max(1u, std::min({FULL_CHUNKS, SEL_TARGET_WGS / ng, vocab / (4 * SEL_THREADS)}));
-        gchunks = std::max(gchunks, (vocab + SEL_CHUNK_MAX - 1) / SEL_CHUNK_MAX);
+        const uint32_t gchunks = sel_gather_chunks(vocab, std::min(FULL_CHUNKS, SEL_TARGET_WGS / ng), SEL_THREADS);
         FullScratch fs{ctx->d_keyA,     ctx->d_idA,      ctx->d_keyB,     ctx->d_idB,        ctx->d_probs,
                        ctx->d_part_max, ctx->d_part_am,  ctx->d_psum,     ctx->d_surv,       ctx->d_full_row,
                        ctx->d_full_arrive, f.chunks,     gchunks,         ctx->d_sel_cnt,    ctx->d_sel_mass,

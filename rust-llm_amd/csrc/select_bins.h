@@ -44,6 +44,34 @@ constexpr uint32_t SEL_GROUP_LOG = 12;
 constexpr uint32_t SEL_GROUP = 1u << SEL_GROUP_LOG;
 constexpr uint32_t SEL_GROUP_CAP = 2 * SEL_GROUP;  // most elements of a group (no bin above SEL_GROUP)
 constexpr uint32_t SEL_GROUPS = 64;                // most groups of a row
+// k_full_gather reads a row in chunks of whole float4, each of at least one and
+// of at most SEL_CHUNK_MAX elements (a window bitmap of 8 KiB; the last chunk
+// takes the row's vocab % 4 besides).
+constexpr uint32_t SEL_CHUNK_MAX = 65536;
+constexpr uint32_t SEL_MIN_VOCAB = 4;
+
+// Whether a row takes the selection path (full_select.h): it keeps the head of
+// the descending order, by top-k (top_k < vocab), or by top-p alone over the
+// whole vocabulary (with min-p on it tries the min-p path). A vocabulary
+// without a float4 to read is left to k_full_rest.
+RL_HD inline bool sel_takes(float temperature, uint64_t top_k, float top_p, float min_p, uint32_t vocab) {
+    const bool by_k = top_k != 0 && top_k < vocab;
+    return vocab >= SEL_MIN_VOCAB && temperature > 0.0f && (by_k || (top_p < 1.0f && !(min_p > 0.0f)));
+}
+
+// The gather's chunks a row when `want` are wished for (vocab >= SEL_MIN_VOCAB):
+// each of at least a float4 for each of a workgroup's `threads`, or one chunk,
+// and as many as SEL_CHUNK_MAX asks for.
+RL_HD inline uint32_t sel_gather_chunks(uint32_t vocab, uint32_t want, uint32_t threads) {
+    const uint32_t most = vocab / (4 * threads), least = (vocab + SEL_CHUNK_MAX - 1) / SEL_CHUNK_MAX;
+    const uint32_t c = want < most ? want : most;
+    return c > least ? c : least;
+}
+
+// Chunk c of n items split into `chunks`: [chunk_lo(c), chunk_lo(c + 1)).
+// Callers split a row's float4 (n <= 2^19, the vocabulary being at most 2^21)
+// into at most FULL_CHUNKS, so n * c fits 32 bits.
+RL_HD inline uint32_t chunk_lo(uint32_t n, uint32_t c, uint32_t chunks) { return n * c / chunks; }
 
 RL_HD inline uint32_t sel_bits(float v) {
 #ifdef __HIP_DEVICE_COMPILE__

@@ -105,6 +105,21 @@ def test_vocabulary_edges(device, V):
     check(device, "V %d top-p" % V, logits, st[8:8 + rows], rng)
 
 
+@pytest.mark.parametrize("V", [1, 2, 3, 4, 5, 7, 8, 9])
+def test_smallest_vocabularies(device, V):
+    """Below four ids a row has no float4 to gather (it is sorted whole); from
+    four on it is gathered from one or two, top-p alone, one row and several."""
+    for rows in (1, 6):
+        print("select smallest", V, rows, flush=True)
+        rng = np.random.default_rng(20 + V + rows)
+        logits = rng.normal(0.0, 1.0, (rows, V)).astype(np.float32)
+        st = [R.sampling(0.9, 0, tp, 0.0, 1.1, 64, r) for r, tp in enumerate((0.9, 0.5, 0.99, 0.0, 0.999, 0.3))][:rows]
+        win = rng.integers(0, V + 2, (rows, 64)).astype(np.uint32)
+        got, want = run_case(device, logits, st, win, np.full(rows, 3, np.uint32),
+                             rng.random(rows).astype(np.float32), "own", max_window=64)
+        assert_rows_match("V %d" % V, got, want, st)
+
+
 @pytest.mark.parametrize("rows", [1, 3, 70, 300])
 def test_rows_beside_other_paths(device, rows):
     print("select mixed", rows, flush=True)

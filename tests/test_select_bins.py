@@ -17,6 +17,8 @@ def lib():
     p = ctypes.c_void_p
     L.sel_bins.argtypes = [p, ctypes.c_float, ctypes.c_uint64, p, p, p]
     L.sel_interval.argtypes = [ctypes.c_double, ctypes.c_uint32, ctypes.c_float, p, p]
+    L.sel_takes_row.argtypes = [ctypes.c_float, ctypes.c_uint64, ctypes.c_float, ctypes.c_float, ctypes.c_uint32]
+    L.sel_chunks.argtypes = [ctypes.c_uint32, ctypes.c_uint32, p, p]
     return L
 
 
@@ -68,3 +70,29 @@ def test_the_interval_holds_the_target_for_sums_in_any_order(lib):
                 t = float(np.float32(top_p)) * seq
                 assert lo.value <= t <= hi.value
                 assert hi.value - lo.value <= 1e-9 * max(abs(t), 1e-300) or t == 0.0
+
+
+def test_every_chunk_of_a_row_it_takes_can_be_read(lib):
+    """A chunk clamps its reads to its own last float4, so it must have one;
+    its window bitmap holds SEL_CHUNK_MAX elements and the row's vocab % 4."""
+    fewest, most = ctypes.c_uint32(), ctypes.c_uint32()
+    rng = np.random.default_rng(14)
+    vocabs = list(range(1, 9000)) + [2**21 - d for d in range(5)] + rng.integers(9000, 2**21, 3000).tolist()
+    vocabs += [65536 * m + d for m in range(1, 32) for d in range(-5, 6)]
+    for V in vocabs:
+        takes = [lib.sel_takes_row(1.0, 0, 0.9, 0.0, V), lib.sel_takes_row(1.0, 65, 1.0, 0.0, V),
+                 lib.sel_takes_row(0.5, 1, 0.9, 0.1, V)]
+        assert takes == [V >= 4, V > 65, V >= 4], V
+        if not any(takes):
+            continue
+        for want in (64, 32, 5, 1):
+            c = lib.sel_chunks(V, want, ctypes.byref(fewest), ctypes.byref(most))
+            assert 1 <= c <= 64 and fewest.value >= 1 and most.value <= 65536 + 3, (V, want, c)
+
+
+def test_rows_it_does_not_take(lib):
+    nan = float("nan")
+    for t, k, top_p, min_p in ((0.0, 0, 0.9, 0.0), (-1.0, 100, 0.9, 0.0), (nan, 100, 0.9, 0.0), (1.0, 0, 1.0, 0.0),
+                               (1.0, 0, nan, 0.0), (1.0, 5000, 1.0, 0.0), (1.0, 2**40, 1.5, 0.0), (1.0, 0, 0.9, 0.05)):
+        assert lib.sel_takes_row(t, k, top_p, min_p, 5000) == 0, (t, k, top_p, min_p)
+    assert lib.sel_takes_row(1.0, 0, 0.9, nan, 5000) == 1  # min_p > 0 does not hold
