@@ -587,7 +587,13 @@ __device__ __forceinline__ uint32_t stat_shift(uint32_t k) {
     return sh;
 }
 
-// grid (slots), REST_THREADS: the rows the kernels before left (done == 0).
+// grid (slots), REST_THREADS: the rows the kernels before left (done == 0). VAL:
+// some may have their values counted (k_full_pass). The value finish is kept
+// apart from the sort: in one kernel, with the row's settings in registers
+// across both, the sort's loops spilled more and every sorted row took 2-3 %
+// longer (256 x 151936 ties with candidates 411 us a call, 407 with the
+// settings loaded anew, 401 without VAL besides).
+template <bool VAL>
 __global__ __launch_bounds__(REST_THREADS) void k_full_rest(RowIO a, FullScratch f) {
     __shared__ union {
         RestLds rest;
@@ -599,16 +605,15 @@ __global__ __launch_bounds__(REST_THREADS) void k_full_rest(RowIO a, FullScratch
     if (st.done) return;
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / WAVE;
     const uint32_t row = a.rows ? a.rows[slot] : a.row0 + slot;
-    if (st.values != 0) {
-        if (finish_values(a, f, slot, row, a.settings[row], st.values, window_len(a, row), (RL_LDS ValLds *)&L_.val,
-                          &st.M))
-            return;
-        __syncthreads();  // its LDS is free
+    if constexpr (VAL) {
+        if (st.values != 0) {
+            if (finish_values(a, f, slot, row, a.settings[row], st.values, window_len(a, row), (RL_LDS ValLds *)&L_.val,
+                              &st.M))
+                return;
+            __syncthreads();  // its LDS is free
+        }
+        asm volatile("" ::: "memory");  // the sort loads its settings anew
     }
-    // The sort loads its settings anew: kept in registers across the value
-    // finish they cost the sort's loops spills, and every sorted row 2-3 %
-    // (256 x 151936 ties with candidates 411 us a call, 401 loaded here).
-    asm volatile("" ::: "memory");
     const rl_sampling s = a.settings[row];
     const uint32_t V = a.vocab;
     const uint32_t k = full_k(s, V);

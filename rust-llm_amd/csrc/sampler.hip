@@ -606,7 +606,7 @@ int rl_sampler_sample_rows(rl_sampler_ctx *ctx, const float *logits, uint64_t ro
             hipLaunchKernelGGL(vec ? k_full_gather<true> : k_full_gather<false>, ggrid, dim3(SEL_THREADS), 0, st, f, fs);
             hipLaunchKernelGGL(k_full_head, dim3(head_wgs, ng), dim3(SEL_THREADS), 0, st, f, fs);
         }
-        hipLaunchKernelGGL(k_full_rest, dim3(ng), dim3(REST_THREADS), 0, st, f, fs);
+        hipLaunchKernelGGL(val ? k_full_rest<true> : k_full_rest<false>, dim3(ng), dim3(REST_THREADS), 0, st, f, fs);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return hip_fail(e, "full-path kernels");
     }
