@@ -406,7 +406,7 @@ __device__ __forceinline__ bool finish_block(const RowIO &a, uint32_t row, const
         // The draw, while the other waves write the candidates.
         float cum = 0.0f;
         uint32_t pick = kept - 1;
-        for (uint32_t b0 = 0; b0 < kept && !(cum > u); b0 += WAVE) {
+        for (uint32_t b0 = 0; b0 < kept; b0 += WAVE) {
             const float q = b0 + tid < kept ? sp[b0 + tid] : 0.0f;
             uint32_t i = 0;
             for (; i < WAVE && b0 + i < kept; i += 4) {
@@ -420,6 +420,7 @@ __device__ __forceinline__ bool finish_block(const RowIO &a, uint32_t row, const
                 do cum += read_lane_f32(q, i++);
                 while (!(cum > u));
                 pick = b0 + i - 1;
+                break;
             }
         }
         if (tid == 0) {
