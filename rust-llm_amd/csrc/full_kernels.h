@@ -49,13 +49,14 @@ struct FullScratch {
     uint32_t *keyA, *idA, *keyB, *idB;  // [slot][vocab] k_full_rest: the sort's passes (keyA: counts first, chunk_counts)
     float *probs;                       // [slot][vocab] k_full_rest: p when the candidates are not returned
     float *part_max;                    // [slot][chunk] k_full_pass: the chunk's maximum
-    uint64_t *part_am;                  // [slot][chunk] k_full_pass: candidates listed << 32 | lowest +inf id
+    uint64_t *part_am;                  // [slot][chunk] k_full_pass: candidates listed (a selection row: 1 when
+                                        // its logits are not on the bf16 grid) << 32 | lowest +inf id
     double *psum;                       // [slot][chunk] k_full_pass: its mass
     uint64_t *surv;                     // [slot][SURV_CAP] min-p candidates (composites), a region per chunk
     FullRow *row;                       // [slot]
     uint32_t *arrive;                   // [slot] workgroups done; zero between kernels
     // The selection path (full_select.h).
-    uint32_t pass_chunks, gather_chunks;  // the grids of k_full_pass and k_full_gather
+    uint32_t pass_chunks, gather_chunks, head_wgs;  // the grids of k_full_pass, k_full_gather and k_full_head
     uint32_t *sel_cnt;                  // [slot][SEL_BINS] elements per bin; zero between calls
     uint32_t *sel_mass;                 // [slot][SEL_BINS] their mass (SEL_MASS_ONE); zero between calls
     uint32_t *sel_off;                  // [slot][SEL_GROUPS + 1] where each group starts
@@ -104,9 +105,11 @@ __device__ __forceinline__ bool small_eligible(const rl_sampling &s, uint32_t V)
     return s.min_p > 0.0f && full_k(s, V) == V && s.temperature > 0.0f;
 }
 
-// Whether a row takes the selection path.
-__host__ __device__ inline bool select_eligible(const rl_sampling &s, uint32_t V) {
-    return sel_takes(s.temperature, s.top_k, s.top_p, s.min_p, V);
+// sel_takes for a row of a launch with selection rows. (Written out: through a
+// shared function the compiler laid k_full_gather out otherwise, and 256 rows
+// took 59 us in it for 54.)
+__device__ __forceinline__ bool select_eligible(const rl_sampling &s, uint32_t V) {
+    return s.temperature > 0.0f && (full_k(s, V) < V || (s.top_p < 1.0f && !(s.min_p > 0.0f)));
 }
 
 // A value row's counts of each value in a chunk: VAL_BINS / 2 words of two. The
@@ -476,10 +479,12 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
     __shared__ uint64_t cbuf[PASS_CAND];  // this chunk's candidates, filtered by its maximum at the end
     __shared__ uint32_t sh_cn, sh_cover;
     __shared__ uint32_t red_cnt[FULL_CHUNKS];   // the finisher: each chunk's listed candidates
-    // The chunk's bins: a selection row's counts and masses, or its values'.
-    __shared__ uint32_t bins[SEL ? 2 * SEL_BINS : VAL ? VAL_BINS : 1];
-    static_assert(2 * SEL_BINS >= VAL_BINS, "the values' bins fit the selection's");
-    uint32_t *const bin_cnt = bins, *const bin_mass = bins + (SEL ? SEL_BINS : 0);
+    // The chunk's bins: a selection row's counts and masses, each followed by a
+    // slot a thread for a common value, or its values'.
+    constexpr uint32_t SEL_SLOTS = SEL_BINS + FULL_THREADS;
+    __shared__ uint32_t bins[SEL ? 2 * SEL_SLOTS : VAL ? VAL_BINS : 1];
+    static_assert(2 * SEL_SLOTS >= VAL_BINS, "the values' bins fit the selection's");
+    uint32_t *const bin_cnt = bins, *const bin_mass = bins + (SEL ? SEL_SLOTS : 0);
     const uint32_t slot = blockIdx.y, chunk = blockIdx.x;
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / WAVE;
     const uint32_t row = a.rows ? a.rows[slot] : a.row0 + slot;
@@ -571,7 +576,7 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
         ref = wave_maxnum_f32(ref);
         if (lane == 0) red_m[wave] = ref;
         if (select)
-            for (uint32_t i = tid; i < SEL_BINS; i += FULL_THREADS) {
+            for (uint32_t i = tid; i < SEL_SLOTS; i += FULL_THREADS) {
                 bin_cnt[i] = 0;
                 bin_mass[i] = 0;
             }
@@ -662,13 +667,20 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
             cbuf[at++] = composite(total_key(value_at(e)), e);
         }
     };
-    // Counts element x into its bin (select rows).
-    auto count = [&](float x) {
+    // Counts element x into its bin (select rows). A value that many of a wave's
+    // elements share (tied, its bits in tie) would queue the lanes on one LDS
+    // address; each thread counts it in a slot of its own then (256 x 151936
+    // constant logits: 261 us in the pass without). off_grid: this wave's
+    // elements are not on the bf16 grid.
+    uint32_t tie = 0;
+    bool tied = false, off_grid = false;
+    auto mass_parts = [&](float edge) { return (uint32_t)(SEL_MASS_ONE * __builtin_amdgcn_exp2f(-edge * c2)); };
+    auto count = [&](float x, bool slots) {
         float edge;
-        const uint32_t b = sel_bin(x, ref, &edge);
+        uint32_t b = sel_bin(x, ref, &edge);
+        if (slots) b = __float_as_uint(x) == tie ? SEL_BINS + tid : b;
         __hip_atomic_fetch_add((RL_LDS uint32_t *)&bin_cnt[b], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        __hip_atomic_fetch_add((RL_LDS uint32_t *)&bin_mass[b],
-                               (uint32_t)(SEL_MASS_ONE * __builtin_amdgcn_exp2f(-edge * c2)), __ATOMIC_RELAXED,
+        __hip_atomic_fetch_add((RL_LDS uint32_t *)&bin_mass[b], mass_parts(edge), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_WORKGROUP);
     };
     // Counts element x's value; false when it has no bin.
@@ -752,11 +764,34 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
         }
         if constexpr (SEL) {
             if (select) {
+                if (b == q0) {
+                    // From the wave's first elements: a quarter of them off
+                    // the grid; neighbours that are equal, and then the
+                    // commonest of eight.
+                    const uint32_t w = __float_as_uint(A[0].x);
+                    off_grid = __popcll(ballot((w & 0xFFFFu) != 0)) >= WAVE / 4;
+                    if (__popcll(ballot(A[0].x == A[0].y)) >= 4) {
+                        uint32_t best = WAVE / 8 - 1;
+#pragma unroll 1
+                        for (uint32_t i = 0; i < 8; ++i) {
+                            const uint32_t v = read_lane_u32(w, 8 * i), n = (uint32_t)__popcll(ballot(w == v));
+                            if (n > best) {
+                                best = n;
+                                tie = v;
+                                tied = true;
+                            }
+                        }
+                    }
+                }
+                auto count_step = [&](bool slots) {
 #pragma unroll
-                for (uint32_t u = 0; u < PASS_U; ++u)
-                    if (b + u * FULL_THREADS + tid < q1)
+                    for (uint32_t u = 0; u < PASS_U; ++u)
+                        if (b + u * FULL_THREADS + tid < q1)
 #pragma unroll
-                        for (uint32_t c = 0; c < 4; ++c) count(A[u][c]);
+                            for (uint32_t c = 0; c < 4; ++c) count(A[u][c], slots);
+                };
+                if (tied) count_step(true);
+                else count_step(false);
             }
         }
         tmax = uniform_f32(wave_maxnum_f32(tmax));
@@ -834,7 +869,7 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
         if (ok) {
             xe = ((const RL_GLB float *)rowp)[e];
             if (pen && ((bm[(e - e0) >> 5] >> ((e - e0) & 31)) & 1u)) xe = penalize(xe, s.repeat_penalty);
-            if (select) count(xe);
+            if (select) count(xe, false);
         }
         const float tmax = uniform_f32(wave_maxnum_f32(xe));
         if (tmax > m_run) {
@@ -863,6 +898,20 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
         uint32_t fi = first_inf;
         fi = wave_fold_u32(fi, [](uint32_t a, uint32_t b) { return a < b ? a : b; });
         first_inf = fi;
+    }
+    if constexpr (SEL) {
+        if (select) {
+            if (tied) {
+                const uint32_t n = wave_sum_u32(bin_cnt[SEL_BINS + tid]);
+                float edge;
+                const uint32_t b = sel_bin(__uint_as_float(tie), ref, &edge);
+                if (lane == 0) {
+                    atomicAdd(&bin_cnt[b], n);
+                    atomicAdd(&bin_mass[b], n * mass_parts(edge));
+                }
+            }
+            if (lane == 0) red_f[wave] = off_grid ? 1u : 0u;
+        }
     }
     if (lane == 0) {
         red_m[wave] = m_run;
@@ -911,6 +960,8 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
     } else if (sh_cover != 0) {
         nkeep = LIST_OVER;
     }
+    if (SEL && select)
+        for (uint32_t w = 0; w < FULL_WAVES; ++w) nkeep |= red_f[w];
     if (wave == 0) {
         uint32_t fi = 0xFFFFFFFFu;
         for (uint32_t w = 0; w < FULL_WAVES; ++w) fi = min(fi, red_i[w]);

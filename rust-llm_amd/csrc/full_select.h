@@ -600,13 +600,18 @@ struct GatherLds {
 // a tenth of what is left out to spare) passes top_p of the whole. c, m: the
 // counts and masses of the bins SEL_PER tid ..; M: the row's maximum. Sets
 // st.thr, st.count and st.groups and, for a long head, L->pos and L->off; or
-// leaves the row to k_full_rest whole (st.thr SEL_NONE): nothing to leave out,
-// a bin too full to be sorted in LDS (many tied logits), or no mass to go by.
+// leaves the row to k_full_rest whole (st.thr SEL_NONE): a bin too full to be
+// sorted in LDS (many tied logits), a long head on the bf16 grid with few
+// workgroups for it (SEL_GRID_GROUPS), or no mass to go by. Such a
+// row has paid for its bins and two launches: 151936 ids, 40 % of them tied, at
+// top-p 0.9 take 324 us at one row and 427 at 256, against 315 and 381 sorted at
+// once; constant logits 190 and 292 against 186 and 251.
 constexpr uint32_t SEL_PER = 3;
 static_assert(SEL_PER * SEL_THREADS >= SEL_BINS && SEL_BINS % SEL_PER == 0, "the bins over the threads");
 
 __device__ __forceinline__ void pick_bins(const uint32_t (&c)[SEL_PER], const uint32_t (&m)[SEL_PER], uint32_t V,
-                                          const rl_sampling &s, FullRow &st, RL_LDS GatherLds *L) {
+                                          const rl_sampling &s, bool grid, bool pen, uint32_t head_wgs,
+                                          FullRow &st, RL_LDS GatherLds *L) {
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / WAVE;
     const float c2 = (float)(1.4426950408889634 / (double)s.temperature);
     const uint32_t k = full_k(s, V);
@@ -647,7 +652,8 @@ __device__ __forceinline__ void pick_bins(const uint32_t (&c)[SEL_PER], const ui
     const double y1 = y0 + yi;
     y0 = y1 - ysum;
     const double tp = (double)s.top_p;
-    const double want = by_k ? (double)k : fmax(tp + 0.1 * (1.0 - tp), 0.0) * yt;
+    // A top_p <= 0 is met by the first candidate.
+    const double want = by_k ? (double)k : fmax(tp + 0.1 * (1.0 - tp), 0.1) * yt;
     if (y0 < want && y1 >= want) {
         double t = y0;
         uint32_t n = c0, bins = 0;  // this thread's bins up to the one that reaches it
@@ -664,24 +670,28 @@ __device__ __forceinline__ void pick_bins(const uint32_t (&c)[SEL_PER], const ui
     }
     __syncthreads();
     const uint32_t last = L->last, count = L->count;
-    if (last == 0 || count == V) return;
+    if (last == 0) return;
     if (count > SEL_FIN_CAP) {
+        if (grid && count > (pen ? SEL_GRID_GROUPS_PEN : SEL_GRID_GROUPS) * SEL_GROUP * head_wgs) return;
         uint32_t run = c0, most = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < SEL_PER; ++i) most = max(most, tid * SEL_PER + i < last ? c[i] : 0u);
+        most = wave_fold_u32(most, [](uint32_t p, uint32_t q) { return p > q ? p : q; });
+        if (lane == 0) atomicMax((uint32_t *)&L->most, most);
+        __syncthreads();
+        if (L->most > SEL_GROUP) return;
 #pragma unroll
         for (uint32_t i = 0; i < SEL_PER; ++i) {
             const uint32_t b = tid * SEL_PER + i;
             if (b < SEL_BINS) L->pos[b] = run;
             if (b < last && c[i] != 0) {
-                most = max(most, c[i]);
                 if ((run >> SEL_GROUP_LOG) < SEL_GROUPS) atomicMin((uint32_t *)&L->off[run >> SEL_GROUP_LOG], run);
                 atomicMax((uint32_t *)&L->groups, (run >> SEL_GROUP_LOG) + 1);
             }
             run += c[i];
         }
-        most = wave_fold_u32(most, [](uint32_t p, uint32_t q) { return p > q ? p : q; });
-        if (lane == 0) atomicMax((uint32_t *)&L->most, most);
         __syncthreads();
-        if (L->most > SEL_GROUP || L->groups > SEL_GROUPS) return;
+        if (L->groups > SEL_GROUPS) return;
     }
     st.thr = last - 1;
     st.count = count;
@@ -727,6 +737,7 @@ __global__ __launch_bounds__(SEL_THREADS) void k_full_gather(RowIO a, FullScratc
     }
     const uint32_t lc = min(lane, C1 - 1);
     const float pm = ((const RL_GLB float *)f.part_max)[slot * C1 + lc];
+    const uint64_t rec = ((const RL_GLB uint64_t *)f.part_am)[slot * C1 + lc];
     const float R = ((const RL_GLB float *)&f.row[slot].R)[0];
     uint32_t c[SEL_PER], m[SEL_PER];
 #pragma unroll
@@ -778,7 +789,7 @@ __global__ __launch_bounds__(SEL_THREADS) void k_full_gather(RowIO a, FullScratc
 #pragma unroll
     for (uint32_t i = 0; i < SEL_PER; ++i)
         if (tid * SEL_PER + i >= SEL_BINS) c[i] = m[i] = 0;
-    if (finite) pick_bins(c, m, V, s, st, L);
+    if (finite) pick_bins(c, m, V, s, ballot((rec >> 32) != 0) == 0, pen, f.head_wgs, st, L);
     if (chunk == 0) {
         if (tid == 0) {
             f.row[slot] = st;

@@ -62,6 +62,10 @@ Path plan_row(const rl_sampling &s, uint32_t vocab) {
     return Path::Full;
 }
 
+bool takes_selection(const rl_sampling &s, uint32_t vocab) {
+    return sel_takes(s.temperature, s.top_k, s.top_p, s.min_p, vocab);
+}
+
 uint64_t row_cand_need(const rl_sampling &s, uint32_t vocab) {
     if (s.temperature <= 0.0f) return 1;
     if (s.top_k == 0 || s.top_k >= vocab) return vocab;
@@ -388,7 +392,7 @@ int rl_sampler_configure(rl_sampler_ctx *ctx, const rl_sampling *settings, uint3
         (p == Path::Greedy ? ctx->greedy_rows : p == Path::Stream ? ctx->stream_rows : ctx->full_rows).push_back(r);
         if (p == Path::Full) {
             const uint32_t before = ctx->select_upto.empty() ? 0u : ctx->select_upto.back();
-            ctx->select_upto.push_back(before + (select_eligible(settings[r], ctx->vocab) ? 1u : 0u));
+            ctx->select_upto.push_back(before + (takes_selection(settings[r], ctx->vocab) ? 1u : 0u));
         }
         need = std::max(need, row_cand_need(settings[r], ctx->vocab));
         ctx->need_upto.push_back(need);
@@ -585,10 +589,13 @@ int rl_sampler_sample_rows(rl_sampler_ctx *ctx, const float *logits, uint64_t ro
         // start late (sixteen waves each): 16 x 248320 at top-k 100 47 us a
         // call with 512, 42 with 256, 43 with 192.
         const uint32_t gchunks = sel_gather_chunks(vocab, std::min(FULL_CHUNKS, SEL_TARGET_WGS / ng), SEL_THREADS);
+        // A row's workgroups share a long head's groups, while rows are few.
+        const uint32_t head_wgs = std::max(1u, std::min(MAX_CHUNKS, SEL_HEAD_WGS / ng));
         FullScratch fs{ctx->d_keyA,     ctx->d_idA,      ctx->d_keyB,     ctx->d_idB,        ctx->d_probs,
                        ctx->d_part_max, ctx->d_part_am,  ctx->d_psum,     ctx->d_surv,       ctx->d_full_row,
-                       ctx->d_full_arrive, f.chunks,     gchunks,         ctx->d_sel_cnt,    ctx->d_sel_mass,
-                       ctx->d_sel_off,  ctx->d_sel_fill, ctx->d_sel_n,    ctx->d_sel_tail,   ctx->d_sel_rec};
+                       ctx->d_full_arrive, f.chunks,     gchunks,         head_wgs,          ctx->d_sel_cnt,
+                       ctx->d_sel_mass, ctx->d_sel_off,  ctx->d_sel_fill, ctx->d_sel_n,      ctx->d_sel_tail,
+                       ctx->d_sel_rec};
         const dim3 cgrid(f.chunks, ng), ggrid(gchunks, ng);
         const size_t pass_lds = k_full_pass_lds_bytes(vocab, f.chunks);
         // Rows that try the min-p path may be finished from their values'
@@ -601,8 +608,6 @@ int rl_sampler_sample_rows(rl_sampler_ctx *ctx, const float *logits, uint64_t ro
                                       : (val ? k_full_pass<false, false, true> : k_full_pass<false, false, false>));
         hipLaunchKernelGGL(pass, cgrid, dim3(FULL_THREADS), pass_lds, st, f, fs);
         if (nsel) {
-            // A row's workgroups share a long head's groups, while rows are few.
-            const uint32_t head_wgs = std::max(1u, std::min(MAX_CHUNKS, SEL_HEAD_WGS / ng));
             hipLaunchKernelGGL(vec ? k_full_gather<true> : k_full_gather<false>, ggrid, dim3(SEL_THREADS), 0, st, f, fs);
             hipLaunchKernelGGL(k_full_head, dim3(head_wgs, ng), dim3(SEL_THREADS), 0, st, f, fs);
         }

@@ -44,6 +44,18 @@ constexpr uint32_t SEL_GROUP_LOG = 12;
 constexpr uint32_t SEL_GROUP = 1u << SEL_GROUP_LOG;
 constexpr uint32_t SEL_GROUP_CAP = 2 * SEL_GROUP;  // most elements of a group (no bin above SEL_GROUP)
 constexpr uint32_t SEL_GROUPS = 64;                // most groups of a row
+// The most groups per workgroup of k_full_head for which a row on the bf16 grid
+// is collected. Its few distinct values crowd the sort's buckets, so a group
+// takes a sorting network's time (75-85 us against 20), while k_full_rest sorts
+// such a row in two passes instead of four: 151936 N(0, 2^2) ids at top-p 0.9,
+// nine groups a row, take 303 us collected at 64 rows (four workgroups a row)
+// against 510 sorted whole, and 832 against 543 at 256 (one); nearly flat ones,
+// 34 groups, 238 against 439 at 8 rows, but 691 against 450 at 64 and 2110
+// against 481 at 256. Rows off the grid gain to the end (256 nearly flat rows
+// 830 against 982).
+// Penalised logits leave the grid, and the whole sort then takes its four
+// passes too (256 nearly flat rows 1065 against 2115 collected).
+constexpr uint32_t SEL_GRID_GROUPS = 3, SEL_GRID_GROUPS_PEN = 12;
 // k_full_gather reads a row in chunks of whole float4, each of at least one and
 // of at most SEL_CHUNK_MAX elements (a window bitmap of 8 KiB; the last chunk
 // takes the row's vocab % 4 besides).
@@ -51,12 +63,13 @@ constexpr uint32_t SEL_CHUNK_MAX = 65536;
 constexpr uint32_t SEL_MIN_VOCAB = 4;
 
 // Whether a row takes the selection path (full_select.h): it keeps the head of
-// the descending order, by top-k (top_k < vocab), or by top-p alone over the
-// whole vocabulary (with min-p on it tries the min-p path). A vocabulary
-// without a float4 to read is left to k_full_rest.
-RL_HD inline bool sel_takes(float temperature, uint64_t top_k, float top_p, float min_p, uint32_t vocab) {
-    const bool by_k = top_k != 0 && top_k < vocab;
-    return vocab >= SEL_MIN_VOCAB && temperature > 0.0f && (by_k || (top_p < 1.0f && !(min_p > 0.0f)));
+// the descending order, by top-k (top_k < V), or by top-p alone over the whole
+// vocabulary (with min-p on it tries the min-p path). The host's rule; a
+// vocabulary without a float4 to read launches no selection kernel, and its
+// rows are left to k_full_rest.
+inline bool sel_takes(float temperature, uint64_t top_k, float top_p, float min_p, uint32_t V) {
+    const bool by_k = top_k != 0 && top_k < V;
+    return V >= SEL_MIN_VOCAB && temperature > 0.0f && (by_k || (top_p < 1.0f && !(min_p > 0.0f)));
 }
 
 // The gather's chunks a row when `want` are wished for (vocab >= SEL_MIN_VOCAB):

@@ -8,6 +8,7 @@ import pytest
 
 import rl_sampler as R
 from test_gpu_long_windows import assert_rows_match, run_case
+from test_gpu_values import to_grid
 
 pytestmark = pytest.mark.gpu
 
@@ -161,3 +162,32 @@ def test_a_context_is_reused(device):
             torch.cuda.synchronize()
             res.append((tok.tolist(), kept.tolist(), used.tolist()))
         assert res[0] == res[1], (kind, res)
+
+
+@pytest.mark.parametrize("top_p,penalty", [(0.9, 1.0), (0.5, 1.0), (0.9, 1.1), (-0.5, 1.0)])
+def test_long_heads_on_the_grid_at_many_rows(device, top_p, penalty):
+    """One workgroup a row: heads of bf16 logits past three groups of 4096 are
+    sorted whole, shorter ones and penalised ones collected; a top_p below 0
+    keeps the first candidate."""
+    print("select grid", top_p, penalty, flush=True)
+    rng = np.random.default_rng(31)
+    V, rows = 20004, 256
+    x = np.repeat(to_grid(rng.normal(0.0, 0.01, (4, V))), rows // 4, axis=0)
+    x[:: 3, ::2] = 0.015625  # every second id tied, in and above the head
+    st = [R.sampling(1.0, 0, top_p, 0.0, penalty, 64, r) for r in range(rows)]
+    check(device, "grid", x, st, rng)
+
+
+def test_heads_that_leave_nothing_out(device):
+    """top-k one below the vocabulary and top-p next to 1: the bins reach the
+    row's end, with ties there and without."""
+    print("select whole rows", flush=True)
+    rng = np.random.default_rng(32)
+    for V in (3001, 50004):
+        x = rng.normal(0.0, 2.0, (6, V)).astype(np.float32)
+        x[1::2, rng.random(V) < 0.02] = -9.0
+        x[4, :] = 0.5
+        st = [R.sampling(1.0, V - 1, 1.0, 0.0, 1.1, 64, 1), R.sampling(1.0, V - 1, 0.9, 0.0, 1.0, 0, 2),
+              R.sampling(1.0, 0, 0.9999999, 0.0, 1.0, 0, 3), R.sampling(2.0, V - 2, 1.0, 0.001, 1.0, 0, 4),
+              R.sampling(1.0, V - 1, 1.0, 0.0, 1.0, 0, 5), R.sampling(0.1, 0, 0.9999999, 0.0, 1.0, 0, 6)]
+        check(device, "whole %d" % V, x, st, rng)
