@@ -461,9 +461,9 @@ __host__ __device__ inline size_t k_full_pass_lds_bytes(uint32_t vocab, uint32_t
 // k_full_gather, which takes such rows from there.
 // With VAL (the call takes no candidates and a chunk's counts fit 16 bits), a
 // row that tries the min-p path with top-p on and that a sample of 64 logits
-// calls nearly flat and on the bf16 grid (half of the sample within min-p's
-// reach of its maximum, so the min-p path would find far more survivors than it
-// finishes) has its values counted instead: each chunk leaves its counts in
+// calls nearly flat and on the bf16 grid (half of the sample's finite ones
+// within min-p's reach of its maximum, so the min-p path would find far more
+// survivors than it finishes) has its values counted instead: each chunk leaves its counts in
 // chunk_counts and lists the elements without a bin, for k_full_rest.
 template <bool VEC, bool SEL, bool VAL>
 __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScratch f) {
@@ -541,9 +541,13 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
     }
     // Every wave takes the same sample of the row, so that all its chunks
     // decide alike without hearing of each other; it is waited for with the
-    // step (ahead of the step's loads it cost a min-p call 0.5 us).
+    // step (ahead of the step's loads it cost a min-p call 0.5 us). It is
+    // taken at eight places of the row: a vocabulary's first ids (control and
+    // byte tokens) say little of the others (one bf16 zipf row with its first
+    // 64 ids flat 39 us by its values, 17 as the min-p row it is), and 64
+    // places cost 128 rows 0.9 us.
     float smp = 0.0f;
-    if constexpr (VAL) smp = ((const RL_GLB float *)rowp)[min(lane, V - 1)];
+    if constexpr (VAL) smp = ((const RL_GLB float *)rowp)[min((lane / 8) * (V / 8) + V / 16 + (lane & 7u), V - 1)];
     // The row's settings and window length, needed from here on (the
     // barrier keeps the wait for them below the step's loads).
     __builtin_amdgcn_sched_barrier(0);
@@ -603,15 +607,18 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScra
     uint32_t hot = 0;       // the bits of a value that is counted in registers, this lane's share:
     uint32_t hot_n = 0;
     if (VAL && mass && s.top_p < 1.0f && ballot((__float_as_uint(smp) & 0xFFFFu) != 0) == 0) {
-        const float top = uniform_f32(wave_maxnum_f32(smp)), mag = uniform_f32(wave_maxnum_f32(fabsf(smp)));
-        if (2 * (uint32_t)__popcll(ballot((smp - top) * c2 >= zthr)) >= WAVE && mag < __builtin_inff()) {
+        // Ids that are ruled out (-inf) count for nothing.
+        const bool fin = fabsf(smp) < __builtin_inff();
+        const float top = uniform_f32(wave_maxnum_f32(smp)), mag = uniform_f32(wave_maxnum_f32(fin ? fabsf(smp) : 0.0f));
+        const uint32_t reach = (uint32_t)__popcll(ballot((smp - top) * c2 >= zthr));
+        if (2 * reach >= (uint32_t)__popcll(ballot(fin)) && reach >= 4) {
             vlo = val_window(__float_as_uint(mag));
             // A value that many elements share (a padded or tied part of the
             // vocabulary) would queue a wave's lanes on one LDS counter: the
             // commonest of sixteen of the sample's is counted in registers.
             uint32_t best = 0;
             for (uint32_t i = 0; i < 16; ++i) {
-                const uint32_t v = read_lane_u32(__float_as_uint(smp), i);
+                const uint32_t v = read_lane_u32(__float_as_uint(smp), 4 * i);
                 const uint32_t n = (uint32_t)__popcll(ballot(__float_as_uint(smp) == v));
                 if (n > best && val_bin(v, vlo) != VAL_NONE) {
                     best = n;

@@ -134,6 +134,34 @@ def test_the_draw_at_every_part_of_the_row(device):
     check(ctx, device, "draw", x, [SETTINGS[1]] * rows, win, np.full(rows, 64, np.uint32), u)
 
 
+def test_samples_that_mislead(device):
+    """The rule looks at 64 ids, eight at each of eight places: rows flat there
+    and peaked elsewhere, peaked there and flat elsewhere, ruled out there, tied
+    there, and with few to too many ids off the grid elsewhere."""
+    print("values misled", flush=True)
+    rng = np.random.default_rng(12)
+    V, rows = 20004, 13
+    at = ((np.arange(64) // 8) * (V // 8) + V // 16 + (np.arange(64) & 7))
+    x = logits_of("ties", rng, rows, V)
+    x[0] = to_grid(rng.normal(0.0, 3.0, V))
+    x[1] = rng.normal(0.0, 3.0, V).astype(np.float32)
+    x[2] = rng.normal(0.0, 0.01, V).astype(np.float32)
+    x[:3, at] = -0.0234375
+    x[3, at] = to_grid(rng.normal(0.0, 3.0, 64))
+    x[4, at] = -np.inf
+    x[5, at[3:]] = -np.inf
+    x[6, at[8:]] = -np.inf
+    x[7, at] = -3.0
+    others = np.setdiff1d(np.arange(V), at)
+    for r, n in enumerate((500, 1023, 1024, 1025, V // 2)):
+        x[8 + r, rng.permutation(others)[:n]] = rng.normal(0.0, 0.01, n).astype(np.float32)
+    ctx = R.DeviceSampler(rows, V, max_window=64)
+    win = rng.integers(0, V, (rows, 64)).astype(np.uint32)
+    for st in SETTINGS[:3]:
+        check(ctx, device, "misled", x, [st] * rows, win, np.full(rows, 64, np.uint32),
+              rng.random(rows).astype(np.float32))
+
+
 def test_beside_other_paths(device):
     """Value rows, min-p rows, selection rows and stream rows in one call, twice."""
     print("values mixed", flush=True)
