@@ -34,7 +34,7 @@ struct HeadLds {
 // fp at the group's place in the list (the first k candidates), with
 // device-scope stores for the workgroup that finishes the row, and its share of
 // the list's statistics to f.sel_rec.
-__device__ __forceinline__ void sort_groups(const FullScratch &f, uint32_t slot, RL_LDS HeadLds *L, const FullRow &st,
+__device__ __forceinline__ void sort_groups(const SelScratch &f, uint32_t slot, RL_LDS HeadLds *L, const FullRow &st,
                                             uint32_t V, uint32_t k, float min_p, const TempScale &tscale,
                                             const LdsExpTable &etab, uint32_t *fid, float *fp) {
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / WAVE;
@@ -83,7 +83,7 @@ __device__ __forceinline__ void sort_groups(const FullScratch &f, uint32_t slot,
 // first k candidates in order, CS groups' records their statistics, tail the
 // sum of every other p (0 for top-k). Returns false (no output final) when the
 // row is not decided here.
-__device__ __forceinline__ bool finish_long(const RowIO &a, const FullScratch &f, uint32_t slot, uint32_t row,
+__device__ __forceinline__ bool finish_long(const RowIO &a, const SelScratch &f, uint32_t slot, uint32_t row,
                                             const rl_sampling &s, const FullRow &st, uint32_t k, double tail,
                                             RL_LDS HeadLds *L, uint32_t *fid, float *fp) {
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / WAVE;
@@ -199,7 +199,7 @@ __device__ __forceinline__ bool finish_long(const RowIO &a, const FullScratch &f
 // short head is the first workgroup's; a long one is sorted by all of the
 // row's, the last of which finishes it. Also clears the bins of every row that
 // was counted into them, for the next call.
-__global__ __launch_bounds__(SEL_THREADS) void k_full_head(RowIO a, FullScratch f) {
+__global__ __launch_bounds__(SEL_THREADS) void k_full_head(RowIO a, SelScratch f) {
     __shared__ union {
         HeadLds h;
         FinishLds fin;

@@ -55,7 +55,11 @@ struct FullScratch {
     uint64_t *surv;                     // [slot][SURV_CAP] min-p candidates (composites), a region per chunk
     FullRow *row;                       // [slot]
     uint32_t *arrive;                   // [slot] workgroups done; zero between kernels
-    // The selection path (full_select.h).
+};
+
+// The selection path's (full_select.h), for its own kernels: a call without
+// selection rows launches with the arguments it needs.
+struct SelScratch : FullScratch {
     uint32_t pass_chunks, gather_chunks, head_wgs;  // the grids of k_full_pass, k_full_gather and k_full_head
     uint32_t *sel_cnt;                  // [slot][SEL_BINS] elements per bin; zero between calls
     uint32_t *sel_mass;                 // [slot][SEL_BINS] their mass (SEL_MASS_ONE); zero between calls
@@ -465,8 +469,10 @@ __host__ __device__ inline size_t k_full_pass_lds_bytes(uint32_t vocab, uint32_t
 // within min-p's reach of its maximum, so the min-p path would find far more
 // survivors than it finishes) has its values counted instead: each chunk leaves its counts in
 // chunk_counts and lists the elements without a bin, for k_full_rest.
+template <bool SEL>
+using PassScratch = typename std::conditional<SEL, SelScratch, FullScratch>::type;
 template <bool VEC, bool SEL, bool VAL>
-__global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, FullScratch f) {
+__global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, PassScratch<SEL> f) {
     extern __shared__ __align__(16) uint8_t smem[];
     RL_LDS uint32_t *bm = (RL_LDS uint32_t *)smem;  // window ids in this chunk, one bit per element
     __shared__ float red_m[FULL_WAVES];

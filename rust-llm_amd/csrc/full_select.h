@@ -547,7 +547,7 @@ __device__ __forceinline__ bool finish_selected(const RowIO &a, uint32_t row, co
 
 // A short head (k_full_head, one workgroup): the chunks' elements and tails,
 // the sort and the finish. Returns false when the row is not decided.
-__device__ __forceinline__ bool finish_short(const RowIO &a, const FullScratch &f, uint32_t slot, uint32_t row,
+__device__ __forceinline__ bool finish_short(const RowIO &a, const SelScratch &f, uint32_t slot, uint32_t row,
                                              const rl_sampling &s, const FullRow &st, RL_LDS FinishLds *L) {
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid / WAVE;
     const uint32_t C = f.gather_chunks, n4 = a.vocab / 4;
@@ -706,7 +706,7 @@ __device__ __forceinline__ void pick_bins(const uint32_t (&c)[SEL_PER], const ui
 // the cache and two scans, while its logits are in flight) rather than wait
 // for the pass to have one workgroup do it after all the others.
 template <bool VEC>
-__global__ __launch_bounds__(SEL_THREADS) void k_full_gather(RowIO a, FullScratch f) {
+__global__ __launch_bounds__(SEL_THREADS) void k_full_gather(RowIO a, SelScratch f) {
     __shared__ GatherLds L_;
     RL_LDS GatherLds *L = (RL_LDS GatherLds *)&L_;
     const uint32_t slot = blockIdx.y, chunk = blockIdx.x;

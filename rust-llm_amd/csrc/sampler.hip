@@ -591,25 +591,27 @@ int rl_sampler_sample_rows(rl_sampler_ctx *ctx, const float *logits, uint64_t ro
         const uint32_t gchunks = sel_gather_chunks(vocab, std::min(FULL_CHUNKS, SEL_TARGET_WGS / ng), SEL_THREADS);
         // A row's workgroups share a long head's groups, while rows are few.
         const uint32_t head_wgs = std::max(1u, std::min(MAX_CHUNKS, SEL_HEAD_WGS / ng));
-        FullScratch fs{ctx->d_keyA,     ctx->d_idA,      ctx->d_keyB,     ctx->d_idB,        ctx->d_probs,
-                       ctx->d_part_max, ctx->d_part_am,  ctx->d_psum,     ctx->d_surv,       ctx->d_full_row,
-                       ctx->d_full_arrive, f.chunks,     gchunks,         head_wgs,          ctx->d_sel_cnt,
-                       ctx->d_sel_mass, ctx->d_sel_off,  ctx->d_sel_fill, ctx->d_sel_n,      ctx->d_sel_tail,
-                       ctx->d_sel_rec};
+        const FullScratch fs{ctx->d_keyA,     ctx->d_idA,     ctx->d_keyB, ctx->d_idB,  ctx->d_probs,
+                             ctx->d_part_max, ctx->d_part_am, ctx->d_psum, ctx->d_surv, ctx->d_full_row,
+                             ctx->d_full_arrive};
+        const SelScratch ss{fs, f.chunks, gchunks, head_wgs, ctx->d_sel_cnt, ctx->d_sel_mass, ctx->d_sel_off,
+                            ctx->d_sel_fill, ctx->d_sel_n, ctx->d_sel_tail, ctx->d_sel_rec};
         const dim3 cgrid(f.chunks, ng), ggrid(gchunks, ng);
         const size_t pass_lds = k_full_pass_lds_bytes(vocab, f.chunks);
         // Rows that try the min-p path may be finished from their values'
         // counts (full_values.h): in calls that take no candidates, in chunks
         // whose counts fit 16 bits and whose tables fit the row's scratch.
         const bool val = !f.out_ids && nsel < ng && vocab >= 4096 && vocab / f.chunks < 65528;
-        const auto pass = vec ? (nsel ? (val ? k_full_pass<true, true, true> : k_full_pass<true, true, false>)
-                                      : (val ? k_full_pass<true, false, true> : k_full_pass<true, false, false>))
-                              : (nsel ? (val ? k_full_pass<false, true, true> : k_full_pass<false, true, false>)
-                                      : (val ? k_full_pass<false, false, true> : k_full_pass<false, false, false>));
-        hipLaunchKernelGGL(pass, cgrid, dim3(FULL_THREADS), pass_lds, st, f, fs);
         if (nsel) {
-            hipLaunchKernelGGL(vec ? k_full_gather<true> : k_full_gather<false>, ggrid, dim3(SEL_THREADS), 0, st, f, fs);
-            hipLaunchKernelGGL(k_full_head, dim3(head_wgs, ng), dim3(SEL_THREADS), 0, st, f, fs);
+            const auto pass = vec ? (val ? k_full_pass<true, true, true> : k_full_pass<true, true, false>)
+                                  : (val ? k_full_pass<false, true, true> : k_full_pass<false, true, false>);
+            hipLaunchKernelGGL(pass, cgrid, dim3(FULL_THREADS), pass_lds, st, f, ss);
+            hipLaunchKernelGGL(vec ? k_full_gather<true> : k_full_gather<false>, ggrid, dim3(SEL_THREADS), 0, st, f, ss);
+            hipLaunchKernelGGL(k_full_head, dim3(head_wgs, ng), dim3(SEL_THREADS), 0, st, f, ss);
+        } else {
+            const auto pass = vec ? (val ? k_full_pass<true, false, true> : k_full_pass<true, false, false>)
+                                  : (val ? k_full_pass<false, false, true> : k_full_pass<false, false, false>);
+            hipLaunchKernelGGL(pass, cgrid, dim3(FULL_THREADS), pass_lds, st, f, fs);
         }
         hipLaunchKernelGGL(val ? k_full_rest<true> : k_full_rest<false>, dim3(ng), dim3(REST_THREADS), 0, st, f, fs);
         const hipError_t e = hipGetLastError();
