@@ -465,9 +465,9 @@ __host__ __device__ inline size_t k_full_pass_lds_bytes(uint32_t vocab, uint32_t
 // k_full_gather, which takes such rows from there.
 // With VAL (the call takes no candidates and a chunk's counts fit 16 bits), a
 // row that tries the min-p path with top-p on and that a sample of 64 logits
-// calls nearly flat and on the bf16 grid (half of the sample's finite ones
-// within min-p's reach of its maximum, so the min-p path would find far more
-// survivors than it finishes) has its values counted instead: each chunk leaves its counts in
+// calls nearly flat and on the bf16 grid (half of the sample's finite ones, or
+// three quarters, within min-p's reach of its maximum, so the min-p path would
+// find far more survivors than it finishes) has its values counted instead: each chunk leaves its counts in
 // chunk_counts and lists the elements without a bin, for k_full_rest.
 template <bool SEL>
 using PassScratch = typename std::conditional<SEL, SelScratch, FullScratch>::type;
@@ -617,7 +617,12 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, PassScra
         const bool fin = fabsf(smp) < __builtin_inff();
         const float top = uniform_f32(wave_maxnum_f32(smp)), mag = uniform_f32(wave_maxnum_f32(fin ? fabsf(smp) : 0.0f));
         const uint32_t reach = (uint32_t)__popcll(ballot((smp - top) * c2 >= zthr));
-        if (2 * reach >= (uint32_t)__popcll(ballot(fin)) && reach >= 4) {
+        // In few chunks each is likely to hold one of the row's peaks, if it
+        // has any, and the min-p path then finishes rows whose bulk is as wide
+        // as a bf16 N(0, 2^2) at temperature 1.2 (14 x 6506 with 16 peaks: 43 us
+        // by its values, 15 by min-p); in many it falls to the sort.
+        const uint32_t n_fin = (uint32_t)__popcll(ballot(fin));
+        if ((C <= 8 ? 4 * reach >= 3 * n_fin : 2 * reach >= n_fin) && reach >= 3 * WAVE / 8) {
             vlo = val_window(__float_as_uint(mag));
             // A value that many elements share (a padded or tied part of the
             // vocabulary) would queue a wave's lanes on one LDS counter: the
