@@ -4,7 +4,7 @@
 // A short head is one workgroup's work in LDS (finish_short): reading,
 // sorting, cutting and drawing 930 elements takes about 10 us, the barriers and
 // the draw's chain of additions most of it. A long head is sorted in groups of
-// 4096 to 8192 elements, spread over the row's workgroups; the last of them to
+// some 4096 elements, spread over the row's workgroups; the last of them to
 // finish goes through the whole list. Heads of tens of thousands of elements
 // are what flat rows (a high temperature, top_p 0.99) leave.
 #pragma once

@@ -808,7 +808,7 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, PassScra
 #pragma unroll
                             for (uint32_t c = 0; c < 4; ++c) count(A[u][c], slots);
                 };
-                if (tied) count_step(true);
+                if (__builtin_expect(tied, 0)) count_step(true);
                 else count_step(false);
             }
         }
@@ -919,7 +919,7 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, PassScra
     }
     if constexpr (SEL) {
         if (select) {
-            if (tied) {
+            if (__builtin_expect(tied, 0)) {
                 const uint32_t n = wave_sum_u32(bin_cnt[SEL_BINS + tid]);
                 float edge;
                 const uint32_t b = sel_bin(__uint_as_float(tie), ref, &edge);

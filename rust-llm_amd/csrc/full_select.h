@@ -435,23 +435,38 @@ __device__ __forceinline__ bool finish_selected(const RowIO &a, uint32_t row, co
     // in order, every wave alike.
     const bool exact = emin > 1000 || list < mul_pow2(1.0 - 0x1p-30, 30 + emin);
     RL_LDS const uint32_t *pw = (RL_LDS const uint32_t *)L->p;
-    const auto never = [](double) { return false; };
+    // The first of the first n sums to reach `stop`, or n, and that sum: one
+    // wave's work (by every wave alike, four to a SIMD, 26 x 7552 at temperature
+    // 0.52, top-k 1904, took 119 us a call, 79 so; wave_walk's passes took 20
+    // less, and their code cost a head of 100 that never runs it 0.3).
+    auto replay = [&](uint32_t n, double stop, double *sum) {
+        if (wave == 0) {
+            double c = 0.0;
+            const uint32_t j = seq_walk<53>(pw, n, [stop](double x) { return x >= stop; }, c);
+            if (lane == 0) {
+                L->sh_at = c;
+                L->sh_hit = j;
+            }
+        }
+        __syncthreads();
+        const uint32_t j = L->sh_hit;
+        *sum = L->sh_at;
+        __syncthreads();
+        return j;
+    };
     uint32_t m = kk;
     double total = list;
     bool have_total = exact;
     if (s.top_p < 1.0f) {
         double t_lo, t_hi;
         if (by_k) {
-            if (!exact) {
-                list = 0.0;
-                seq_walk<53>(pw, kk, never, list);
-            }
+            if (__builtin_expect(!exact, 0)) replay(kk, __builtin_inf(), &list);
             t_lo = t_hi = (double)s.top_p * list;  // the candidates' mass, in order
         } else {
             sel_target_interval(tail + list, V, s.top_p, &t_lo, &t_hi);
         }
         uint32_t j;
-        if (exact) {
+        if (__builtin_expect(exact, 1)) {
             double c = before;
             uint32_t hit = 0xFFFFFFFFu;
 #pragma unroll
@@ -472,8 +487,7 @@ __device__ __forceinline__ bool finish_selected(const RowIO &a, uint32_t row, co
             __syncthreads();
             total = L->sh_at;
         } else {
-            total = 0.0;
-            j = seq_walk<53>(pw, kk, [t_lo](double c) { return c >= t_lo; }, total);
+            j = replay(kk, t_lo, &total);
             if (j >= kk) j = 0xFFFFFFFFu;
         }
         if (j == 0xFFFFFFFFu) {
@@ -511,14 +525,13 @@ __device__ __forceinline__ bool finish_selected(const RowIO &a, uint32_t row, co
         m = w;
     }
     if (!have_total) {
-        if (exact) {
+        if (__builtin_expect(exact, 1)) {
             double part = 0.0;
 #pragma unroll
             for (uint32_t i = 0; i < PER; ++i) part += i < per && tid * per + i < m ? (double)p[i] : 0.0;
             block_exclusive<SEL_THREADS, double>(part, (RL_LDS double *)L->red_d, &total);
         } else {
-            total = 0.0;
-            seq_walk<53>(pw, m, never, total);
+            replay(m, __builtin_inf(), &total);
         }
     }
     const float inv = (float)(1.0 / total);
@@ -602,7 +615,8 @@ struct GatherLds {
 // st.thr, st.count and st.groups and, for a long head, L->pos and L->off; or
 // leaves the row to k_full_rest whole (st.thr SEL_NONE): a bin too full to be
 // sorted in LDS (many tied logits), a long head on the bf16 grid with few
-// workgroups for it (SEL_GRID_GROUPS), or no mass to go by. Such a
+// workgroups for it (SEL_GRID_SHARE), ties in a small vocabulary
+// (SEL_SMALL_VOCAB), or no mass to go by. Such a
 // row has paid for its bins and two launches: 151936 ids, 40 % of them tied, at
 // top-p 0.9 take 324 us at one row and 427 at 256, against 315 and 381 sorted at
 // once; constant logits 190 and 292 against 186 and 251.
@@ -671,15 +685,20 @@ __device__ __forceinline__ void pick_bins(const uint32_t (&c)[SEL_PER], const ui
     __syncthreads();
     const uint32_t last = L->last, count = L->count;
     if (last == 0) return;
-    if (count > SEL_FIN_CAP) {
-        if (grid && count > (pen ? SEL_GRID_GROUPS_PEN : SEL_GRID_GROUPS) * SEL_GROUP * head_wgs) return;
-        uint32_t run = c0, most = 0;
+    const bool small = V < SEL_SMALL_VOCAB, big = count > SEL_FIN_CAP;
+    if (big && grid && (pen ? SEL_GRID_SHARE_PEN : SEL_GRID_SHARE) * (count / head_wgs) > 2 * V) return;
+    if (small && count == V) return;
+    if (big || small) {
+        uint32_t most = 0;
 #pragma unroll
         for (uint32_t i = 0; i < SEL_PER; ++i) most = max(most, tid * SEL_PER + i < last ? c[i] : 0u);
         most = wave_fold_u32(most, [](uint32_t p, uint32_t q) { return p > q ? p : q; });
         if (lane == 0) atomicMax((uint32_t *)&L->most, most);
         __syncthreads();
-        if (L->most > SEL_GROUP) return;
+        if (L->most > (small ? SEL_SMALL_TIES : SEL_GROUP)) return;
+    }
+    if (big) {
+        uint32_t run = c0;
 #pragma unroll
         for (uint32_t i = 0; i < SEL_PER; ++i) {
             const uint32_t b = tid * SEL_PER + i;

@@ -39,23 +39,30 @@ constexpr uint32_t SEL_SAMPLE = 1024;            // logits R is taken from
 constexpr uint32_t SEL_NONE = 0xFFFFFFFFu;       // FullRow::thr of a row that is not collected
 // Collected elements are sorted a group at a time: a group is the bins whose
 // first element's rank shares its upper bits, at most SEL_GROUP elements and
-// the rest of a last bin.
+// the rest of a last bin. No bin of a collected head holds more than SEL_GROUP:
+// a fuller one could reach past the next group, which no bin would then start.
 constexpr uint32_t SEL_GROUP_LOG = 12;
 constexpr uint32_t SEL_GROUP = 1u << SEL_GROUP_LOG;
 constexpr uint32_t SEL_GROUP_CAP = 2 * SEL_GROUP;  // most elements of a group (no bin above SEL_GROUP)
 constexpr uint32_t SEL_GROUPS = 64;                // most groups of a row
-// The most groups per workgroup of k_full_head for which a row on the bf16 grid
-// is collected. Its few distinct values crowd the sort's buckets, so a group
-// takes a sorting network's time (75-85 us against 20), while k_full_rest sorts
-// such a row in two passes instead of four: 151936 N(0, 2^2) ids at top-p 0.9,
-// nine groups a row, take 303 us collected at 64 rows (four workgroups a row)
-// against 510 sorted whole, and 832 against 543 at 256 (one); nearly flat ones,
-// 34 groups, 238 against 439 at 8 rows, but 691 against 450 at 64 and 2110
-// against 481 at 256. Rows off the grid gain to the end (256 nearly flat rows
-// 830 against 982).
-// Penalised logits leave the grid, and the whole sort then takes its four
-// passes too (256 nearly flat rows 1065 against 2115 collected).
-constexpr uint32_t SEL_GRID_GROUPS = 3, SEL_GRID_GROUPS_PEN = 12;
+// A head on the bf16 grid that is too long for one workgroup's LDS is collected
+// when this many times its elements, shared by the row's workgroups of
+// k_full_head, are no more than twice the vocabulary. Its few distinct values crowd
+// the sort's buckets, so a group takes a sorting network's time (75-85 us
+// against 20), while k_full_rest sorts such a row in two passes instead of four:
+// 151936 N(0, 2^2) ids at top-p 0.9, nine groups a row, take 303 us collected at
+// 64 rows (four workgroups a row) against 510 sorted whole, and 832 against 543
+// at 256 (one); nearly flat ones, 34 groups, 238 against 439 at 8 rows, but 691
+// against 450 at 64 and 2110 against 481 at 256. Rows off the grid gain to the
+// end (256 nearly flat rows 830 against 982). Penalised logits leave the grid,
+// and the whole sort then takes its four passes too (256 nearly flat rows 1065
+// against 2115 collected, N(0, 2^2) 1066 against 840).
+constexpr uint32_t SEL_GRID_SHARE = 12, SEL_GRID_SHARE_PEN = 3;
+// Below this vocabulary, where the whole sort takes 45-100 us, a head with a bin
+// of more than SEL_SMALL_TIES is left to it: the bin's ties crowd the sort's
+// buckets (4 x 2854 ids, 40 % tied, at top-p 0.95: 54 us sorted, 82 collected);
+// and so is a head of every id (37 x 15680: 116 us sorted, 174 collected).
+constexpr uint32_t SEL_SMALL_VOCAB = 16384, SEL_SMALL_TIES = 512;
 // k_full_gather reads a row in chunks of whole float4, each of at least one and
 // of at most SEL_CHUNK_MAX elements (a window bitmap of 8 KiB; the last chunk
 // takes the row's vocab % 4 besides).
