@@ -29,10 +29,10 @@ struct FullRow {
     float M;           // the f32::max fold of the penalised row
     uint32_t done;     // the row is finished (no finite maximum, the min-p path, or the selection path)
     uint32_t thr;      // the last bin k_full_gather collects, or SEL_NONE
-    float R;           // the bins' reference value
     uint32_t count;    // elements in bins 0..thr
+    float R;           // the bins' reference value
+    uint32_t binned;   // the row was counted into bins (they are cleared by k_full_head): 1, or 2 on the bf16 grid
     uint32_t groups;   // groups they are sorted in
-    uint32_t binned;   // the row was counted into bins (they are cleared by k_full_head)
     uint32_t values;   // the window its values were counted in (value_bins.h), or 0
 };
 
@@ -49,8 +49,7 @@ struct FullScratch {
     uint32_t *keyA, *idA, *keyB, *idB;  // [slot][vocab] k_full_rest: the sort's passes (keyA: counts first, chunk_counts)
     float *probs;                       // [slot][vocab] k_full_rest: p when the candidates are not returned
     float *part_max;                    // [slot][chunk] k_full_pass: the chunk's maximum
-    uint64_t *part_am;                  // [slot][chunk] k_full_pass: candidates listed (a selection row: 1 when
-                                        // its logits are not on the bf16 grid) << 32 | lowest +inf id
+    uint64_t *part_am;                  // [slot][chunk] k_full_pass: candidates listed << 32 | lowest +inf id
     double *psum;                       // [slot][chunk] k_full_pass: its mass
     uint64_t *surv;                     // [slot][SURV_CAP] min-p candidates (composites), a region per chunk
     FullRow *row;                       // [slot]
@@ -529,12 +528,15 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, PassScra
     }
     const uint64_t tab = EXP2_32_TAB[tid & 31u];
     float ref = -__builtin_inff();  // the sample's maximum (SEL)
+    uint32_t ref_bits = 0;
     if constexpr (SEL) {
         static_assert(SEL_SAMPLE == 4 * FULL_THREADS, "four samples a thread");
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) {
             const uint32_t e = k * FULL_THREADS + tid;
-            ref = fmaxf(ref, ((const RL_GLB float *)rowp)[e < V ? e : V - 1]);
+            const float x = ((const RL_GLB float *)rowp)[e < V ? e : V - 1];
+            ref = fmaxf(ref, x);
+            ref_bits |= __float_as_uint(x);
         }
     }
     f32x4 A[PASS_U];
@@ -584,16 +586,24 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, PassScra
     const bool select = SEL && select_eligible(s, V);
     if constexpr (SEL) {
         ref = wave_maxnum_f32(ref);
-        if (lane == 0) red_m[wave] = ref;
+        const bool off_grid = ballot((ref_bits & 0xFFFFu) != 0) != 0;
+        if (lane == 0) {
+            red_m[wave] = ref;
+            red_f[wave] = off_grid ? 1u : 0u;
+        }
         if (select)
-            for (uint32_t i = tid; i < SEL_SLOTS; i += FULL_THREADS) {
+            for (uint32_t i = tid; i < SEL_BINS; i += FULL_THREADS) {
                 bin_cnt[i] = 0;
                 bin_mass[i] = 0;
             }
     }
     __syncthreads();
     if constexpr (SEL) {
-        for (uint32_t w = 0; w < FULL_WAVES; ++w) ref = fmaxf(ref, red_m[w]);
+        ref_bits = 0;  // from here on whether the sample is off the grid
+        for (uint32_t w = 0; w < FULL_WAVES; ++w) {
+            ref = fmaxf(ref, red_m[w]);
+            ref_bits |= red_f[w];
+        }
         // + 0: a reference of -0 would part the two zeros' bins from the rest of the order.
         ref = uniform_f32((ref > -__builtin_inff() && ref < __builtin_inff() ? ref : 0.0f) + 0.0f);
         __syncthreads();  // red_m is written again at the chunk's end
@@ -688,10 +698,9 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, PassScra
     // Counts element x into its bin (select rows). A value that many of a wave's
     // elements share (tied, its bits in tie) would queue the lanes on one LDS
     // address; each thread counts it in a slot of its own then (256 x 151936
-    // constant logits: 261 us in the pass without). off_grid: this wave's
-    // elements are not on the bf16 grid.
+    // constant logits: 261 us in the pass without).
     uint32_t tie = 0;
-    bool tied = false, off_grid = false;
+    bool tied = false;
     auto mass_parts = [&](float edge) { return (uint32_t)(SEL_MASS_ONE * __builtin_amdgcn_exp2f(-edge * c2)); };
     auto count = [&](float x, bool slots) {
         float edge;
@@ -783,12 +792,10 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, PassScra
         if constexpr (SEL) {
             if (select) {
                 if (b == q0) {
-                    // From the wave's first elements: a quarter of them off
-                    // the grid; neighbours that are equal, and then the
-                    // commonest of eight.
-                    const uint32_t w = __float_as_uint(A[0].x);
-                    off_grid = __popcll(ballot((w & 0xFFFFu) != 0)) >= WAVE / 4;
-                    if (__popcll(ballot(A[0].x == A[0].y)) >= 4) {
+                    // From the wave's first elements: neighbours that are
+                    // equal, and then the commonest of eight.
+                    if (__builtin_expect(__popcll(ballot(A[0].x == A[0].y)) >= 4, 0)) {
+                        const uint32_t w = __float_as_uint(A[0].x);
                         uint32_t best = WAVE / 8 - 1;
 #pragma unroll 1
                         for (uint32_t i = 0; i < 8; ++i) {
@@ -799,6 +806,7 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, PassScra
                                 tied = true;
                             }
                         }
+                        bin_cnt[SEL_BINS + tid] = 0;
                     }
                 }
                 auto count_step = [&](bool slots) {
@@ -928,7 +936,6 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, PassScra
                     atomicAdd(&bin_mass[b], n * mass_parts(edge));
                 }
             }
-            if (lane == 0) red_f[wave] = off_grid ? 1u : 0u;
         }
     }
     if (lane == 0) {
@@ -978,8 +985,6 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, PassScra
     } else if (sh_cover != 0) {
         nkeep = LIST_OVER;
     }
-    if (SEL && select)
-        for (uint32_t w = 0; w < FULL_WAVES; ++w) nkeep |= red_f[w];
     if (wave == 0) {
         uint32_t fi = 0xFFFFFFFFu;
         for (uint32_t w = 0; w < FULL_WAVES; ++w) fi = min(fi, red_i[w]);
@@ -1014,7 +1019,10 @@ __global__ __launch_bounds__(FULL_THREADS, 4) void k_full_pass(RowIO a, PassScra
                     __hip_atomic_fetch_add(f.sel_mass + (uint64_t)slot * SEL_BINS + i, bin_mass[i], __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_AGENT);
                 }
-            if (chunk == 0 && tid == 0) f.row[slot].R = ref;
+            if (chunk == 0 && tid == 0) {
+                f.row[slot].R = ref;
+                f.row[slot].binned = ref_bits != 0 ? 1u : 2u;
+            }
             return;
         }
     }

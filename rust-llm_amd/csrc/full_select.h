@@ -756,8 +756,8 @@ __global__ __launch_bounds__(SEL_THREADS) void k_full_gather(RowIO a, SelScratch
     }
     const uint32_t lc = min(lane, C1 - 1);
     const float pm = ((const RL_GLB float *)f.part_max)[slot * C1 + lc];
-    const uint64_t rec = ((const RL_GLB uint64_t *)f.part_am)[slot * C1 + lc];
     const float R = ((const RL_GLB float *)&f.row[slot].R)[0];
+    const uint32_t binned = ((const RL_GLB uint32_t *)&f.row[slot].binned)[0];
     uint32_t c[SEL_PER], m[SEL_PER];
 #pragma unroll
     for (uint32_t i = 0; i < SEL_PER; ++i) {
@@ -802,13 +802,13 @@ __global__ __launch_bounds__(SEL_THREADS) void k_full_gather(RowIO a, SelScratch
     st.M = uniform_f32(wave_maxnum_f32(pm));
     st.thr = SEL_NONE;
     st.R = uniform_f32(R);
-    st.binned = 1;
+    st.binned = uniform_u32(binned);  // and R: what the other chunks may yet read stays as it is
     const bool finite = st.M > -__builtin_inff() && st.M < __builtin_inff();
     st.done = finite ? 0u : 1u;
 #pragma unroll
     for (uint32_t i = 0; i < SEL_PER; ++i)
         if (tid * SEL_PER + i >= SEL_BINS) c[i] = m[i] = 0;
-    if (finite) pick_bins(c, m, V, s, ballot((rec >> 32) != 0) == 0, pen, f.head_wgs, st, L);
+    if (finite) pick_bins(c, m, V, s, st.binned == 2, pen, f.head_wgs, st, L);
     if (chunk == 0) {
         if (tid == 0) {
             f.row[slot] = st;
