@@ -655,17 +655,19 @@ void k_head_dot(const uint4 *__restrict__ wq, const uint32_t *__restrict__ ws, c
 // It reads the tensor as it was uploaded, a row's blocks side by side: in the
 // matrix-core layout a block lies in 15 cache lines shared with 15 other rows
 // (9.3 times the bytes used were read). 2048 tokens of 2560: 14.9 -> 7.2 us,
-// against about 4 for the bytes used; the launch is most of the rest. One wave per (token, block): lane j writes values 4 j .. 4 j +
-// 3 (a wave 1 KiB in one store) from four bytes of ql, four of qh, the
-// sub-block's scale and d. A token at or past `rows` gives a row of NaN: the
+// against about 4 for the bytes used; the launch is most of the rest. One wave
+// per (token, block): lane j writes values 4 j .. 4 j + 3 (a wave 1 KiB in one
+// store) from four bytes of ql, four of qh, the sub-block's scale and d. A token at or past `rows` gives a row of NaN: the
 // reference asserts (forward.rs:1130-1134), which a kernel cannot.
 constexpr int EMBED_THREADS = 256;
 
 // The four bytes at p (2-byte aligned, with four readable bytes after them,
-// in a buffer that starts 4-byte aligned).
+// in a buffer that starts 4-byte aligned). One load of eight bytes, which the
+// type says are aligned to four only.
 __device__ __forceinline__ uint32_t embed_word(const uint8_t *p) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2), aligned(4)));
     const uintptr_t at = reinterpret_cast<uintptr_t>(p);
-    const uint2 w = *reinterpret_cast<const uint2 *>(at & ~(uintptr_t)3);
+    const u32x2 w = *reinterpret_cast<const u32x2 *>(at & ~(uintptr_t)3);
     return __builtin_amdgcn_alignbyte(w.y, w.x, (uint32_t)at & 3u);
 }
 
