@@ -129,23 +129,6 @@ __host__ __device__ inline size_t chunk_bitmap_bytes(uint32_t vocab, uint32_t ch
     return ((size_t)(most + 31) / 32) * 4;
 }
 
-// One wave's lanes with the same 8-bit digit (among the lanes where valid).
-// Per bit: the lane's bit as a 0 / all-ones word, its ballot, and one
-// three-input logic operation per mask half (m & ~(ballot ^ own)), so the
-// select between a ballot and its complement costs no 64-bit arithmetic.
-__device__ __forceinline__ uint64_t match_digit(uint32_t d, bool valid) {
-    const uint64_t v = ballot(valid);
-    uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
-#pragma unroll
-    for (uint32_t b = 0; b < 8; ++b) {
-        const uint32_t own = (uint32_t)((int32_t)(d << (31 - b)) >> 31);  // bit b of d, replicated
-        const uint64_t bb = ballot(own != 0u);
-        lo &= ~((uint32_t)bb ^ own);
-        hi &= ~((uint32_t)(bb >> 32) ^ own);
-    }
-    return ((uint64_t)hi << 32) | lo;
-}
-
 // ----------------------------------------------------------- min-p path ---
 // A row with min-p on and the whole vocabulary as candidates keeps only
 // candidates with p >= min_p (sample.rs:326-340), usually a few. Those are the

@@ -32,7 +32,7 @@
 // sequential sum is the exact sum, and any summation order (an f64 tree)
 // computes it exactly, however many binades the sum crosses on the way.
 //
-// The core (grid, term maps, runs, parities) is plain C++ usable on the host,
+// The core (grid, steps, runs, parities) is plain C++ usable on the host,
 // where a test checks it against sequential loops; the workgroup-wide replay
 // is device code.
 #pragma once
@@ -49,14 +49,6 @@
 #endif
 
 namespace rl {
-
-// Increments are saturated here: far above any segment's capacity (< 2^54).
-constexpr uint64_t SEQ_SAT = 1ull << 60;
-
-RL_HD inline uint64_t sat_add(uint64_t a, uint64_t b) {
-    const uint64_t c = a + b;  // a, b <= SEQ_SAT, so no wrap-around
-    return c > SEQ_SAT ? SEQ_SAT : c;
-}
 
 RL_HD inline uint64_t f64_bits(double d) {
     uint64_t b;
@@ -125,78 +117,6 @@ RL_HD inline SumSegF segf_of(double s) {
     g.n = mul_pow2(s, -g.uexp);
     return g;
 }
-
-// The term map: from parity 0 (1) the term adds i0 (i1) grid steps and leaves
-// parity p0 (p1).
-struct TermMap {
-    uint64_t i0, i1;
-    uint32_t p0, p1;
-};
-
-RL_HD inline TermMap map_identity() { return TermMap{0, 0, 0, 1}; }
-
-// The map of adding the f32 term with bits xb (finite, >= 0) on the grid
-// 2^uexp.
-RL_HD inline TermMap map_of(uint32_t xb, int uexp) {
-    uint32_t m = xb & 0x7FFFFFu;
-    const int ex = (int)((xb >> 23) & 0xFFu);
-    int lsb = -149;  // x = m * 2^lsb
-    if (ex != 0) {
-        m |= 0x800000u;
-        lsb = ex - 150;
-    }
-    if (m == 0) return map_identity();
-    const int sh = lsb - uexp;
-    if (sh >= 0) {  // a multiple of the grid step: added exactly
-        const uint64_t n = sh > 36 ? SEQ_SAT : ((uint64_t)m << sh);
-        const uint32_t b = (uint32_t)(n & 1);
-        return TermMap{n, n, b, b ^ 1u};
-    }
-    const int d = -sh;
-    if (d >= 25) return map_identity();  // below half a step: no effect
-    const uint64_t q = m >> d;
-    const uint32_t rem = m & ((1u << d) - 1u), half = 1u << (d - 1);
-    if (rem != half) {
-        const uint64_t n = q + (rem > half ? 1u : 0u);
-        const uint32_t b = (uint32_t)(n & 1);
-        return TermMap{n, n, b, b ^ 1u};
-    }
-    // An exact tie: round to the even significand, which leaves parity 0.
-    return TermMap{q + (q & 1), q + ((q + 1) & 1), 0u, 0u};
-}
-
-// The grid steps the term adds when it is not an exact tie; *tie is set when
-// it is one (its increment then depends on the parity of the sum).
-RL_HD inline uint64_t inc_of(uint32_t xb, int uexp, bool *tie) {
-    uint32_t m = xb & 0x7FFFFFu;
-    const int ex = (int)((xb >> 23) & 0xFFu);
-    int lsb = -149;
-    if (ex != 0) {
-        m |= 0x800000u;
-        lsb = ex - 150;
-    }
-    *tie = false;
-    const int sh = lsb - uexp;
-    if (sh >= 0) return sh > 36 ? SEQ_SAT : ((uint64_t)m << sh);
-    const int d = -sh;
-    if (d >= 25) return 0;
-    const uint32_t rem = m & ((1u << d) - 1u), half = 1u << (d - 1);
-    *tie = m != 0 && rem == half;
-    return (uint64_t)(m >> d) + (rem > half ? 1u : 0u);
-}
-
-// a, then b.
-RL_HD inline TermMap map_then(const TermMap &a, const TermMap &b) {
-    TermMap c;
-    c.i0 = sat_add(a.i0, a.p0 ? b.i1 : b.i0);
-    c.p0 = a.p0 ? b.p1 : b.p0;
-    c.i1 = sat_add(a.i1, a.p1 ? b.i1 : b.i0);
-    c.p1 = a.p1 ? b.p1 : b.p0;
-    return c;
-}
-
-RL_HD inline uint64_t map_inc(const TermMap &t, uint32_t parity) { return parity ? t.i1 : t.i0; }
-RL_HD inline uint32_t map_parity(const TermMap &t, uint32_t parity) { return parity ? t.p1 : t.p0; }
 
 // One IEEE addition in precision P of a P-bit value and an f32 term.
 template <int P>
