@@ -31,11 +31,13 @@ typedef struct rl_head rl_head;
 /* Uploads a Q6_K weight tensor of `rows` rows of `k` values (ggml layout: each
  * row is ceil(k/256) blocks of 210 bytes, `ql[128] qh[64] scales[16] d:f16`;
  * q6k_bytes must be rows * ceil(k/256) * 210) from HOST memory, repacks it on
- * the device into the layout the head kernel streams (same byte count; the
- * uploaded form stays beside it for rl_head_embed_rows), and sizes the activation scratch for up to `max_batch` rows per call. Replaces
- * the memory-mapped tensor view the reference's head reads (`model.token_embd`,
- * forward.rs:934; TensorView, crates/llm-core/src/gguf.rs:190-197).
- * Synchronous. */
+ * the device into the layout the head kernel streams (same byte count), and
+ * sizes the activation scratch for up to `max_batch` rows per call. The uploaded
+ * form stays beside the repacked one for rl_head_embed_rows, so a handle holds
+ * the tensor twice whether or not rows are looked up: 2 x 521 MB at 248320 rows
+ * of 2560. Replaces the memory-mapped tensor view the reference's head reads
+ * (`model.token_embd`, forward.rs:934; TensorView,
+ * crates/llm-core/src/gguf.rs:190-197). Synchronous. */
 int rl_head_create(int device, uint32_t k, uint32_t rows, uint32_t max_batch, const void *q6k,
                    uint64_t q6k_bytes, rl_head **out);
 

@@ -1,15 +1,21 @@
 // The FULL device path: rows with top_k == 0, top_k >= vocab or top_k > 64
-// (sample.rs:279-358 over the whole candidate list). Two launches per group
-// of rows:
+// (sample.rs:279-358 over the whole candidate list). Two launches per group of
+// rows, four when some of them take the selection path:
 //
-//   k_full_pass  (chunks x rows)  the one read of every row: the f32::max
-//                                 fold; rows without a finite maximum
-//                                 answered; min-p rows finished from their
-//                                 survivors when the top-p cut is certain
-//   k_full_rest  (rows)           the rows left, one workgroup each
-//                                 (full_rest.h): the candidates sorted, p, the
-//                                 cut, min-p, the total, the draw and the kept
-//                                 candidates
+//   k_full_pass    (chunks x rows)  the one read of every row: the f32::max
+//                                   fold; rows without a finite maximum
+//                                   answered; min-p rows finished from their
+//                                   survivors when the top-p cut is certain;
+//                                   selection rows counted into bins; nearly
+//                                   flat bf16 rows' values counted
+//   k_full_gather,                  the selection rows: their heads collected,
+//   k_full_head                     sorted and finished (full_select.h,
+//                                   full_head.h)
+//   k_full_rest    (rows)           the rows left, one workgroup each: from
+//                                   their values' counts (full_values.h) or
+//                                   sorted whole (full_rest.h): p, the cut,
+//                                   min-p, the total, the draw and the kept
+//                                   candidates
 //
 // The sums are the reference's sequential sums, bit for bit: when every p is a
 // multiple of 2^(e_min - 23) and the mass is below 2^(30 + e_min), every partial
@@ -36,9 +42,10 @@ struct FullRow {
     uint32_t values;   // the window its values were counted in (value_bins.h), or 0
 };
 
-// Most chunks of a row on the full path: one lane of a wave each. A launch with
-// selection rows uses them all while rows are few; the min-p path's rows, whose
-// last chunk goes through every chunk's candidates, are read in MAX_CHUNKS.
+// Most chunks of a row on the full path: one lane of a wave each. A launch of
+// selection rows alone uses them all while rows are few; any other reads its
+// rows in MAX_CHUNKS, since a min-p row's last chunk goes through every chunk's
+// candidates.
 constexpr uint32_t FULL_CHUNKS = 64;
 // Candidates the min-p path collects per row (a superset of the survivors).
 constexpr uint32_t SURV_CAP = 4096;

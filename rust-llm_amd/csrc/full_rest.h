@@ -1,7 +1,9 @@
 // The FULL path's last launch, k_full_rest: one workgroup per row that the
-// kernels before it (k_full_pass, k_full_head) left unfinished. It puts the row's candidates in the reference's
-// order (descending penalised logit, ascending id; sample.rs:279-305) with a
-// stable LSD radix sort whose passes are chosen by one histogram read, computes
+// kernels before it (k_full_pass, k_full_head) left unfinished. A row whose
+// values k_full_pass counted is finished from the counts (full_values.h) when it
+// can be. Any other's candidates are put in the reference's order (descending
+// penalised logit, ascending id; sample.rs:279-305) with a stable LSD radix sort
+// whose passes are chosen by one histogram read; the kernel computes
 // p = exp((l - max) / T) as the last pass writes each candidate in place
 // (:309), takes the mass, the top-p cut, min-p and the normalising total
 // (:307-343), draws against the host's uniform (:349-358) and writes the kept
@@ -12,8 +14,8 @@
 // each further pass (the last writes ids and p, to the candidate outputs when
 // the caller asked for them), a read of p for the per-chunk sums, and a read
 // and write of the kept prefix for the normalisation (the draw reads up to its
-// pick). A row the pass finished exits at once, so a call whose rows all
-// finished in the pass costs one empty launch here.
+// pick). A finished row exits at once, so a call whose rows are all finished
+// costs one empty launch here.
 #pragma once
 #include "full_values.h"
 

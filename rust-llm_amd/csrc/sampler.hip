@@ -571,14 +571,14 @@ int rl_sampler_sample_rows(rl_sampler_ctx *ctx, const float *logits, uint64_t ro
         f.rows = consecutive ? nullptr : ctx->d_full_rows + g0;
         f.row0 = ctx->full_rows[g0];
         // Rows of the group that take the selection path: with any, the pass
-        // counts bins and the gather runs; with no others, few rows are read
-        // in more chunks. With no others the pass takes half the workgroups:
+        // counts bins and the gather and the head run. A group of them alone
+        // is read in up to FULL_CHUNKS chunks a row, by half the workgroups:
         // each ends with its bins' device-scope adds (24 x 151935 at top-p
         // 0.9 52 -> 48 us a call, 40 x 248320 at top-k 100 60 -> 54 with the
         // gather's below, one to four rows the same).
         const uint32_t nsel = ctx->select_upto[g0 + ng - 1] - (g0 ? ctx->select_upto[g0 - 1] : 0u);
         const uint32_t most = nsel == ng ? FULL_CHUNKS : MAX_CHUNKS;
-        // The same holds for few min-p rows, whose last chunk waits for every
+        // Half the workgroups serve few min-p rows better too, whose last chunk waits for every
         // other's record (32 x 151936 at min-p 0.05 28.5 -> 22.5 us a call,
         // 48 29.7 -> 25.5, 96 34.5 -> 29.8; nearly flat rows 4 us less too).
         const uint32_t pass_wgs = nsel == ng || ng <= FEW_FULL_ROWS ? FEW_PASS_WGS : TARGET_WGS;

@@ -3,8 +3,8 @@
 // A row that keeps the head of the descending order (top-k, or top-p over the
 // whole vocabulary) needs only that head sorted. k_full_pass counts its
 // penalised logits into SEL_BINS bins that fall along the order (bin 0 holds
-// the largest), and the row's last chunk picks the bin down to which the head
-// reaches. A bin only decides which elements are collected: the row is then
+// the largest), and every chunk of k_full_gather picks the bin down to which the
+// head reaches. A bin only decides which elements are collected: the row is then
 // finished from the exact values, or left to k_full_rest.
 //
 // The bins are spaced in the distance of a logit from a reference value R (the

@@ -378,7 +378,8 @@ Q6K_BYTES = 210
 
 class DeviceHead:
     """rl_head_create / rl_head_logits: the tied Q6_K output head
-    (forward.rs:932-937) with its weights resident in HBM."""
+    (forward.rs:932-937) with its weights resident in HBM, twice: in the layout
+    the head streams, and as uploaded for embed_into."""
 
     def __init__(self, q6k, k, rows, max_batch=32, device=0):
         import numpy as np
