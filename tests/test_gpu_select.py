@@ -191,3 +191,56 @@ def test_heads_that_leave_nothing_out(device):
               R.sampling(1.0, 0, 0.9999999, 0.0, 1.0, 0, 3), R.sampling(2.0, V - 2, 1.0, 0.001, 1.0, 0, 4),
               R.sampling(1.0, V - 1, 1.0, 0.0, 1.0, 0, 5), R.sampling(0.1, 0, 0.9999999, 0.0, 1.0, 0, 6)]
         check(device, "whole %d" % V, x, st, rng)
+
+
+def test_largest_vocabularies(device):
+    """Eight rows of 2^21 - 1 ids, which the gather reads in chunks of 65536 (and
+    three): short heads, a penalised window at the chunks' edges, and heads on
+    either side of the 64 groups that are collected."""
+    print("select largest", flush=True)
+    rng = np.random.default_rng(33)
+    V, rows = 2**21 - 1, 8
+    x = rng.normal(0.0, 2.0, (rows, V)).astype(np.float32)
+    edges = np.concatenate([np.arange(c * 65536 - 2, c * 65536 + 2) for c in range(1, 16)] + [[V - 4, V - 3, V - 2, V - 1]])
+    x[:, edges] = rng.uniform(9.0, 14.0, (rows, edges.size))
+    for r, n in ((4, 261000), (5, 263500)):   # 255 and 257 ids a bin, far above the others
+        x[r] -= 3000.0
+        x[r, rng.permutation(V)[:n]] = 20.0 - 2.0 ** rng.uniform(-8.0, 7.9, n)
+    win = np.resize(edges, (rows, 64)).astype(np.uint32)
+    st = [R.sampling(0.8, 100, 0.95, 0.0, 1.1, 64, 1), R.sampling(0.7, 0, 0.9, 0.0, 1.2, 64, 2),
+          R.sampling(1.0, 0, 0.5, 0.0, 1.0, 0, 3), R.sampling(1.0, 65, 1.0, 0.0, 1.3, 64, 4),
+          R.sampling(50.0, 261000, 0.999, 0.0, 1.0, 0, 5), R.sampling(50.0, 263500, 0.999, 0.0, 1.0, 0, 6),
+          R.sampling(1.0, 4000, 0.99, 0.0, 1.1, 64, 7), R.sampling(1.0, 0, 0.3, 0.0, 0.9, 64, 8)]
+    got, want = run_case(device, x, st, win, np.full(rows, 64, np.uint32), rng.random(rows).astype(np.float32), "own",
+                         max_window=64)
+    assert_rows_match("largest", got, want, st)
+
+
+def test_many_rows_of_the_largest_vocabulary(device):
+    """256 rows of 2^21 ids: the pass's largest chunks (two a row), whose window
+    bitmap and bins take nearly all of a compute unit's LDS."""
+    import torch
+    import oracle as O
+    from conftest import as_oracle_settings
+    print("select many large rows", flush=True)
+    rng = np.random.default_rng(34)
+    V, rows = 2**21, 256
+    x = rng.normal(0.0, 2.0, (2, V)).astype(np.float32)
+    x[:, rng.permutation(V)[:64]] = rng.uniform(9.0, 14.0, (2, 64))
+    win = rng.integers(0, V, (2, 64)).astype(np.uint32)
+    win[:, :32] = np.argsort(x, axis=1)[:, -32:]
+    wlen, u = np.full(2, 64, np.uint32), np.array([0.3, 0.9], np.float32)
+    st = [R.sampling(0.8, 100, 0.95, 0.0, 1.1, 64, 1), R.sampling(0.7, 0, 0.9, 0.0, 1.2, 64, 2)]
+    want = O.pick_rows(x, [as_oracle_settings(s) for s in st], win, wlen, u, cand_cap=100)
+    ctx = R.DeviceSampler(rows, V, max_window=64)
+    ctx.configure(st * (rows // 2))
+    rep = lambda a: torch.from_numpy(a).to(device).repeat(rows // 2, *([1] * (a.ndim - 1)))
+    tok = torch.zeros(rows, dtype=torch.int32, device=device)
+    kept, used = torch.zeros_like(tok), torch.zeros(rows, dtype=torch.uint8, device=device)
+    ctx.sample_rows(rep(x), rows, V, tok, kept, used, windows=rep(win.view(np.int32)), window_stride=64,
+                    window_len=rep(wlen.view(np.int32)), uniforms=rep(u))
+    torch.cuda.synchronize()
+    for got, name in ((tok, "token"), (kept, "kept"), (used, "used")):
+        assert np.array_equal(got.cpu().numpy().reshape(-1, 2).astype(np.int64),
+                              np.repeat(want[name][None].astype(np.int64), rows // 2, axis=0)), name
+    ctx.close()

@@ -177,3 +177,21 @@ def test_beside_other_paths(device):
     win = rng.integers(0, V, (rows, 64)).astype(np.uint32)
     for _ in range(2):
         check(ctx, device, "mixed", x, settings, win, np.full(rows, 64, np.uint32), rng.random(rows).astype(np.float32))
+
+
+@pytest.mark.parametrize("V", [2096800, 2096895, 2096900, 2**21])
+def test_chunk_counts_at_their_limit(device, V):
+    """One row in 32 chunks: counts of up to 65531 equal values a chunk, two a
+    word, below 2096896 ids, and the sort above; the value that fills the chunks
+    is the one counted in registers, and is not."""
+    print("values limit", V, flush=True)
+    rng = np.random.default_rng(V)
+    at = ((np.arange(64) // 8) * (V // 8) + V // 16 + (np.arange(64) & 7))
+    win = rng.integers(0, V, (1, 64)).astype(np.uint32)
+    ctx = R.DeviceSampler(1, V, max_window=64)
+    for sampled, step in ((0.5, 64), (0.50390625, 1 << 20)):
+        x = np.full((1, V), 0.5, np.float32)
+        x[0, ::step] = 0.498046875
+        x[0, at] = sampled
+        for u in (0.001, 0.5, 0.999):
+            check(ctx, device, "limit", x, [SETTINGS[1]], win, np.full(1, 64, np.uint32), np.array([u], np.float32))
