@@ -456,8 +456,9 @@ __host__ __device__ inline size_t k_full_pass_lds_bytes(uint32_t vocab, uint32_t
 // row that tries the min-p path with top-p on and that a sample of 64 logits
 // calls nearly flat and on the bf16 grid (half of the sample's finite ones, or
 // three quarters, within min-p's reach of its maximum, so the min-p path would
-// find far more survivors than it finishes) has its values counted instead: each chunk leaves its counts in
-// chunk_counts and lists the elements without a bin, for k_full_rest.
+// find far more survivors than it finishes) has its values counted instead:
+// each chunk leaves its counts in chunk_counts and lists the elements without a
+// bin, for k_full_rest.
 template <bool SEL>
 using PassScratch = typename std::conditional<SEL, SelScratch, FullScratch>::type;
 template <bool VEC, bool SEL, bool VAL>

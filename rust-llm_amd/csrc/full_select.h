@@ -18,9 +18,9 @@
 //
 // Before, k_full_rest sorted every such row: four radix passes over the
 // vocabulary on one CU. A call over one row of 248 320 at top-p 0.95 went from
-// 1348 to 37 us, 24 unaligned rows of 151 935 at top-p 0.9 from 897 to 48 us,
-// 16 rows of 248 320 at top-k 100 from 931 to 40 us. What bounds it now: four
-// launches and, in each, one chain of dependent steps (about 11, 9, 10 and 2 us
+// 1347 to 35 us, 24 unaligned rows of 151 935 at top-p 0.9 from 899 to 47 us,
+// 16 rows of 248 320 at top-k 100 from 928 to 40 us. What bounds it now: four
+// launches and, in each, one chain of dependent steps (about 10, 9, 10 and 2 us
 // at one row); the logits' two reads are a small part.
 //
 // Measured and not kept: the finish in the gather's last chunk to arrive (the
@@ -615,11 +615,11 @@ struct GatherLds {
 // st.thr, st.count and st.groups and, for a long head, L->pos and L->off; or
 // leaves the row to k_full_rest whole (st.thr SEL_NONE): a bin too full to be
 // sorted in LDS (many tied logits), a long head on the bf16 grid with few
-// workgroups for it (SEL_GRID_SHARE), ties in a small vocabulary
-// (SEL_SMALL_VOCAB), or no mass to go by. Such a
-// row has paid for its bins and two launches: 151936 ids, 40 % of them tied, at
-// top-p 0.9 take 324 us at one row and 427 at 256, against 315 and 381 sorted at
-// once; constant logits 190 and 292 against 186 and 251.
+// workgroups for it (SEL_GRID_SHARE), ties or every id in a small vocabulary
+// (SEL_SMALL_VOCAB), or no mass to go by. Such a row has paid for its bins and
+// two launches: 151936 ids, 40 % of them tied, at top-p 0.9 take 324 us at one
+// row and 428 at 256, against 315 and 381 sorted at once; constant logits 190
+// and 295 against 186 and 251.
 constexpr uint32_t SEL_PER = 3;
 static_assert(SEL_PER * SEL_THREADS >= SEL_BINS && SEL_BINS % SEL_PER == 0, "the bins over the threads");
 

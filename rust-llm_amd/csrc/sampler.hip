@@ -578,9 +578,10 @@ int rl_sampler_sample_rows(rl_sampler_ctx *ctx, const float *logits, uint64_t ro
         // gather's below, one to four rows the same).
         const uint32_t nsel = ctx->select_upto[g0 + ng - 1] - (g0 ? ctx->select_upto[g0 - 1] : 0u);
         const uint32_t most = nsel == ng ? FULL_CHUNKS : MAX_CHUNKS;
-        // Half the workgroups serve few min-p rows better too, whose last chunk waits for every
-        // other's record (32 x 151936 at min-p 0.05 28.5 -> 22.5 us a call,
-        // 48 29.7 -> 25.5, 96 34.5 -> 29.8; nearly flat rows 4 us less too).
+        // Half the workgroups serve few min-p rows better too, whose last
+        // chunk waits for every other's record (32 x 151936 at min-p 0.05
+        // 28.5 -> 22.5 us a call, 48 29.7 -> 25.5, 96 34.5 -> 29.8; nearly flat
+        // rows 4 us less too).
         const uint32_t pass_wgs = nsel == ng || ng <= FEW_FULL_ROWS ? FEW_PASS_WGS : TARGET_WGS;
         f.chunks = std::max(1u, std::min(most, (pass_wgs + ng - 1) / ng));
         f.chunks = std::min(f.chunks, std::max(1u, vocab / 4096));
