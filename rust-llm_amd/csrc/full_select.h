@@ -18,7 +18,7 @@
 //
 // Before, k_full_rest sorted every such row: four radix passes over the
 // vocabulary on one CU. A call over one row of 248 320 at top-p 0.95 went from
-// 1347 to 35 us, 24 unaligned rows of 151 935 at top-p 0.9 from 899 to 47 us,
+// 1347 to 35 us, 24 unaligned rows of 151 935 at top-p 0.9 from 899 to 47-50 us,
 // 16 rows of 248 320 at top-k 100 from 928 to 40 us. What bounds it now: four
 // launches and, in each, one chain of dependent steps (about 10, 9, 10 and 2 us
 // at one row); the logits' two reads are a small part.
